@@ -27,6 +27,8 @@
 namespace ihip {
 
 static const int64_t CHUNK = 1024;
+// rows from which the delta rule runs in chunks of tokens (dn_rule_128/_256)
+static const int64_t DN_RULE_ROWS = 8;
 
 struct DevLayer {
   uint64_t input_norm = 0, post_norm = 0, q = 0, k = 0, v = 0, o = 0;
@@ -73,7 +75,7 @@ struct ihip_mctx {
   // a sequence starts); the chunk's DeltaNet channels, gates, beta, decay and
   // the rule's output; a gated attention's query+gate rows and its gates
   std::vector<uint64_t> conv, state;
-  uint64_t qkv = 0, z = 0, beta = 0, decay = 0, core = 0, qg = 0, gq = 0;
+  uint64_t qkv = 0, qkv2 = 0, z = 0, beta = 0, decay = 0, core = 0, qg = 0, gq = 0;
   // Gemma 4: the second rotary set's cos/sin, the experts' sum of a row
   uint64_t cs2 = 0, moe = 0;
   // the rotary rows of positions 0 .. cs_rows - 1 (cs_cap allocated), and the
@@ -395,6 +397,18 @@ struct DnConvPrepArgs {
   const float* dt_bias;
   const float* neg_a;
   int32_t kh, vh, dk, dv, channels, kw;
+};
+struct DnRowsArgs {
+  const float* x;
+  float* y;
+  const float* w;
+  float* conv;
+  float* beta;
+  float* decay;
+  float* z;
+  const float* dt_bias;
+  const float* neg_a;
+  int32_t kh, vh, dk, dv, channels, kw, rows, pad;
 };
 struct DnRuleArgs {
   const float* qkv;
@@ -797,7 +811,7 @@ static int deltanet_block(ihip_mctx* s, int l, int64_t n, QCache* qh, bool fused
   const int64_t H = d.hidden, kh = d.lin_key_heads, vh = d.lin_value_heads, dk = d.lin_key_dim,
                 dv = d.lin_value_dim, vd = vh * dv, cd = 2 * kh * dk + vd;
   int rc;
-  uint64_t decay = s->decay;
+  uint64_t decay = s->decay, qkv = s->qkv;
   if (fused) {
     // one row, x the residual: every projection norms it in its staging; the
     // q/k/v channels, z and beta|alpha (one matrix when their types match,
@@ -839,6 +853,16 @@ static int deltanet_block(ihip_mctx* s, int l, int64_t n, QCache* qh, bool fused
                          (float*)s->z, (const float*)L.ldt, (const float*)L.lnega, (int32_t)kh, (int32_t)vh,
                          (int32_t)dk, (int32_t)dv, (int32_t)cd, d.lin_conv};
     if ((rc = launch(m->c, "dn_convprep1", dim3((unsigned)(2 * kh + vh)), dim3(64), &cp))) return rc;
+  } else if (dv <= 256 && d.lin_conv <= 5) {
+    // several rows: every (item, row) on its own, out of place (an item's
+    // channels in a wave; at most 4 kept inputs, which the first block of rows
+    // reads and moves on)
+    DnRowsArgs cp = {(const float*)s->qkv, (float*)s->qkv2, (const float*)L.lconv, (float*)s->conv[l],
+                     (float*)s->beta, (float*)decay, (float*)s->z, (const float*)L.ldt, (const float*)L.lnega,
+                     (int32_t)kh, (int32_t)vh, (int32_t)dk, (int32_t)dv, (int32_t)cd, d.lin_conv, (int32_t)n, 0};
+    if ((rc = launch(m->c, "dn_convprep", dim3((unsigned)(2 * kh + vh), (unsigned)((n + 3) / 4)), dim3(256), &cp)))
+      return rc;
+    qkv = s->qkv2;
   } else {
     DnConvArgs ca = {(float*)s->qkv, (const float*)L.lconv, (float*)s->conv[l], (int32_t)n, (int32_t)cd,
                      d.lin_conv, 0};
@@ -849,10 +873,16 @@ static int deltanet_block(ihip_mctx* s, int l, int64_t n, QCache* qh, bool fused
   }
   // LinGroup (decoder.pas:2457-2463)
   const int32_t group = d.lin_tiled ? 1 : (int32_t)(vh / kh);
-  DnRuleArgs ra = {(const float*)s->qkv, (const float*)s->beta, (const float*)decay, (float*)s->state[l],
+  DnRuleArgs ra = {(const float*)qkv, (const float*)s->beta, (const float*)decay, (float*)s->state[l],
                    (float*)s->core, (int32_t)n, (int32_t)cd, (int32_t)kh, (int32_t)vh, (int32_t)dk,
                    (int32_t)dv, group, 0};
-  if ((rc = launch(m->c, "dn_rule", dim3((unsigned)vh, (unsigned)((dv + 3) / 4)), dim3(256), &ra))) return rc;
+  // from DN_RULE_ROWS rows, one group of 8 tokens, the chunked form
+  if (n >= DN_RULE_ROWS)
+    rc = launch(m->c, dk <= 128 ? "dn_rule_128" : "dn_rule_256", dim3((unsigned)vh, (unsigned)((dv + 7) / 8)),
+                dim3(256), &ra);
+  else
+    rc = launch(m->c, "dn_rule", dim3((unsigned)vh, (unsigned)((dv + 3) / 4)), dim3(256), &ra);
+  if (rc) return rc;
   DnNormArgs na = {(float*)s->core, (const float*)L.lnorm, (const float*)s->z, (double)d.rms_eps,
                    (int32_t)(n * vh), (int32_t)dv};
   if ((rc = launch(m->c, "dn_gatenorm", dim3((unsigned)((n * vh + 3) / 4)), dim3(256), &na))) return rc;
@@ -1759,7 +1789,8 @@ static int context_new(ihip_model* m, int64_t capacity, ihip_mctx** out)
   s->state.assign(d.layers, 0);
   if (m->recurrent) {
     const int64_t lvh = std::max(d.lin_value_heads, 1);
-    if ((rc = dalloc_ctx(s, N * lcd * 4, s->qkv)) || (rc = dalloc_ctx(s, N * lvd * 4, s->z)) ||
+    if ((rc = dalloc_ctx(s, N * lcd * 4, s->qkv)) || (rc = dalloc_ctx(s, N * lcd * 4, s->qkv2)) ||
+        (rc = dalloc_ctx(s, N * lvd * 4, s->z)) ||
         (rc = dalloc_ctx(s, N * lvh * 4, s->beta)) || (rc = dalloc_ctx(s, N * lvh * 4, s->decay)) ||
         (rc = dalloc_ctx(s, N * lvd * 4, s->core)))
       return bad(rc);

@@ -231,6 +231,128 @@ extern "C" __global__ __launch_bounds__(64) void dn_convprep1(DnConvPrepArgs a)
   for (int j = lane; j < a.dv; j += 64) zz[j] = dn_silu(zz[j]);
 }
 
+struct DnRowsArgs {
+  const float* x;      // [rows, channels]: the projected channels
+  float* y;            // [rows, channels]: convolved, silu'd and prepared
+  const float* w;      // [channels, kw]
+  float* conv;         // [channels, kw - 1], moved on
+  float* beta;         // [rows, vh]
+  float* decay;        // [rows, vh]
+  float* z;            // [rows, vh * dv]
+  const float* dt_bias;
+  const float* neg_a;
+  int32_t kh, vh, dk, dv, channels, kw, rows, pad;
+};
+
+// The convolution and DeltaPrep of a prompt chunk in one launch: one wave per
+// (item, row), dn_conv's and dn_prep's arithmetic. A row's convolution reads
+// the kw - 1 rows before it from x, so it writes to y, and every row is
+// computed on its own: (items) x (rows / 4) blocks fill the chip, where a
+// thread per channel walking the rows in order (24 blocks for 6144 channels)
+// waited for a load and a store per row. Bound by silu's double exp and
+// division (two per channel and row in all). Qwen3.5-0.8B's layer, 512 rows of
+// 6144 channels: 256 + 16 us as dn_conv and dn_prep, 33 us as this.
+// The kept inputs are read by the blocks of the first rows alone; the block
+// of row group 0 writes the new ones after its own reads, so no other block
+// meets them half changed.
+extern "C" __global__ __launch_bounds__(256) void dn_convprep(DnRowsArgs a)
+{
+  const int item = blockIdx.x, lane = threadIdx.x & 63;
+  const int t = blockIdx.y * 4 + (threadIdx.x >> 6);
+  const int i = item - 2 * a.kh;
+  const int first = i < 0 ? item * a.dk : 2 * a.kh * a.dk + i * a.dv;
+  const int cnt = i < 0 ? a.dk : a.dv;
+  const int k1 = a.kw - 1;
+  constexpr int NC = DN_MAXK / 64;  // channels per lane (items of up to 256)
+  if (t < a.rows) {
+    float y[NC];
+#pragma unroll
+    for (int u = 0; u < NC; u++) {
+      y[u] = 0.f;
+      const int cc = lane + 64 * u;
+      if (cc >= cnt) continue;
+      const int64_t c = first + cc;
+      float st[DN_MAXKW], w[DN_MAXKW];
+      // input j of the row is row t - k1 + j, or a kept input before the chunk
+#pragma unroll
+      for (int j = 0; j < DN_MAXKW; j++) {
+        const int r = t - k1 + j;
+        st[j] = j > k1 ? 0.f : r >= 0 ? a.x[(int64_t)r * a.channels + c] : a.conv[c * k1 + k1 + r];
+        w[j] = j <= k1 ? a.w[c * a.kw + j] : 0.f;
+      }
+      float wl = w[0], xl = st[0];
+#pragma unroll
+      for (int j = 1; j < DN_MAXKW; j++)
+        if (j == k1) {
+          wl = w[j];
+          xl = st[j];
+        }
+      double acc = (double)wl * (double)xl;
+#pragma unroll
+      for (int j = 0; j < DN_MAXKW; j++)
+        if (j < k1) acc = __builtin_fma((double)w[j], (double)st[j], acc);
+      y[u] = dn_silu((float)acc);
+    }
+    float* yr = a.y + (int64_t)t * a.channels + first;
+    if (i < 0) {
+      double acc = 0;
+#pragma unroll
+      for (int u = 0; u < NC; u++) {
+        const double e = y[u];
+        acc = __builtin_fma(e, e, acc);
+      }
+      acc = wave_sum(acc, 64);
+      const float f = (float)(1.0 / sqrt(acc + 1e-6));
+      const float scale = (float)(1.0 / sqrt((double)a.dk));
+#pragma unroll
+      for (int u = 0; u < NC; u++) {
+        const int cc = lane + 64 * u;
+        if (cc >= cnt) continue;
+        float v = y[u] * f;
+        if (item < a.kh) v = v * scale;
+        yr[cc] = v;
+      }
+    } else {
+#pragma unroll
+      for (int u = 0; u < NC; u++) {
+        const int cc = lane + 64 * u;
+        if (cc < cnt) yr[cc] = y[u];
+      }
+      const int64_t f = (int64_t)t * a.vh + i;
+      if (lane == 0) {
+        a.beta[f] = dn_sigmoid(a.beta[f]);
+        const float x = a.decay[f] + a.dt_bias[i];
+        float sp;
+        if (x > 20) {
+          sp = x;
+        } else {
+          const double e = exp((double)x);
+          sp = e < 1e-6 ? (float)(e - e * e / 2) : (float)log(1.0 + e);
+        }
+        sp = a.neg_a[i] * sp;
+        a.decay[f] = (float)exp((double)sp);
+      }
+      float* zz = a.z + f * a.dv;
+      for (int j = lane; j < a.dv; j += 64) zz[j] = dn_silu(zz[j]);
+    }
+  }
+  // the kept inputs moved on to the chunk's last ones
+  if (blockIdx.y != 0 || k1 == 0) return;
+  __syncthreads();  // rows 0 .. 3 have read the old ones
+  for (int cc = threadIdx.x; cc < cnt; cc += 256) {
+    const int64_t c = first + cc;
+    float st[DN_MAXKW];
+#pragma unroll
+    for (int j = 0; j < DN_MAXKW; j++) {
+      const int r = a.rows - k1 + j;
+      st[j] = j >= k1 ? 0.f : r >= 0 ? a.x[(int64_t)r * a.channels + c] : a.conv[c * k1 + k1 + r];
+    }
+#pragma unroll
+    for (int j = 0; j < DN_MAXKW; j++)
+      if (j < k1) a.conv[c * k1 + j] = st[j];
+  }
+}
+
 struct DnRuleArgs {
   const float* qkv;    // [rows, stride]: [q heads | k heads | v heads]
   const float* beta;   // [rows, vh]
@@ -314,6 +436,135 @@ extern "C" __global__ __launch_bounds__(256) void dn_rule(DnRuleArgs a)
     if (i < a.dk) col[i] = s[m];
   }
 }
+
+// The delta rule of a prompt chunk: dn_rule's arithmetic and sum order, two
+// columns per wave (a column over 32 lanes, NM pairs of values each, lane L
+// holding values 2L and 2L + 1 of every 64: the first level of dn_rule's wave
+// sum is then inside the lane), the tokens' operands staged through LDS in
+// chunks of CT, the next chunk's loads in flight while one is computed.
+// Bound by a token's serial chain (the prediction's wave sum, delta, the
+// column's update), which the next token's loads, one memory round trip a
+// token, stretched in dn_rule: 16 heads of 128 x 128, 512 tokens, 455 us there,
+// 145 us here (190 with each token's output summed on its own).
+template <int NM, int CT>
+__device__ __forceinline__ void dn_rule_chunks(const DnRuleArgs& a)
+{
+  constexpr int W = 64 * NM;         // a token's q (or k) in LDS, zeros past dk
+  constexpr int PRE = CT * 2 * W / 256;
+  __shared__ float sq[2][CT][2][W];  // [buffer][token][q, k]
+  __shared__ float sv[2][CT][8];     // v of the block's 8 columns
+  __shared__ float sg[2][CT][2];     // decay, beta
+  const int t = threadIdx.x, head = blockIdx.x, L = t & 31;
+  const int jl = t >> 5, j = blockIdx.y * 8 + jl;
+  const int kd = a.kh * a.dk, vdw = a.vh * a.dv;
+  const int off = ((head / a.group) % a.kh) * a.dk;
+  float* col = a.state + ((int64_t)head * a.dv + min(j, a.dv - 1)) * a.dk;
+  float s[NM][2];
+#pragma unroll
+  for (int m = 0; m < NM; m++)
+#pragma unroll
+    for (int e = 0; e < 2; e++) {
+      const int i = 64 * m + 2 * L + e;
+      s[m][e] = i < a.dk ? col[i] : 0.f;
+    }
+  // a thread's share of a chunk's operands, in registers until the chunk
+  // before is computed
+  float pre[PRE], pv = 0.f, pg = 0.f;
+  auto load = [&](int t0) __attribute__((always_inline)) {
+#pragma unroll
+    for (int u = 0; u < PRE; u++) {
+      const int e = t + 256 * u, tok = min(t0 + e / (2 * W), a.rows - 1), i = e % W;
+      const int base = (e / W) & 1 ? kd + off : off;
+      pre[u] = i < a.dk ? a.qkv[(int64_t)tok * a.stride + base + i] : 0.f;
+    }
+    if (t < CT * 8) {
+      const int tok = min(t0 + (t >> 3), a.rows - 1);
+      const int c = min((int)blockIdx.y * 8 + (t & 7), a.dv - 1);
+      pv = a.qkv[(int64_t)tok * a.stride + 2 * kd + (int64_t)head * a.dv + c];
+    } else if (t < CT * 10) {
+      const int u = t - CT * 8, tok = min(t0 + (u >> 1), a.rows - 1);
+      pg = ((u & 1) ? a.beta : a.decay)[(int64_t)tok * a.vh + head];
+    }
+  };
+  auto store = [&](int b) __attribute__((always_inline)) {
+#pragma unroll
+    for (int u = 0; u < PRE; u++) (&sq[b][0][0][0])[t + 256 * u] = pre[u];
+    if (t < CT * 8) sv[b][t >> 3][t & 7] = pv;
+    else if (t < CT * 10) (&sg[b][0][0])[t - CT * 8] = pg;
+  };
+  // one token: the state moved on, this lane's part of the output
+  auto token = [&](int buf, int u) __attribute__((always_inline)) -> double {
+    float q[NM][2], k[NM][2];
+#pragma unroll
+    for (int m = 0; m < NM; m++) {
+      const float2 qq = *(const float2*)&sq[buf][u][0][64 * m + 2 * L];
+      const float2 kk = *(const float2*)&sq[buf][u][1][64 * m + 2 * L];
+      q[m][0] = qq.x; q[m][1] = qq.y;
+      k[m][0] = kk.x; k[m][1] = kk.y;
+    }
+    const float v = sv[buf][u][jl], g = sg[buf][u][0], b = sg[buf][u][1];
+    double p0 = 0, p1 = 0;
+#pragma unroll
+    for (int m = 0; m < NM; m++) {
+      s[m][0] = s[m][0] * g;
+      s[m][1] = s[m][1] * g;
+      p0 = __builtin_fma((double)s[m][0], (double)k[m][0], p0);
+      p1 = __builtin_fma((double)s[m][1], (double)k[m][1], p1);
+    }
+    const float pred = (float)wave_sum(p0 + p1, 32);
+    float delta = v - pred;
+    delta = delta * b;
+    double o0 = 0, o1 = 0;
+#pragma unroll
+    for (int m = 0; m < NM; m++) {
+      const float w0 = k[m][0] * delta, w1 = k[m][1] * delta;
+      s[m][0] = s[m][0] + w0;
+      s[m][1] = s[m][1] + w1;
+      o0 = __builtin_fma((double)s[m][0], (double)q[m][0], o0);
+      o1 = __builtin_fma((double)s[m][1], (double)q[m][1], o1);
+    }
+    return o0 + o1;
+  };
+  load(0);
+  store(0);
+  __syncthreads();
+  int buf = 0;
+  for (int t0 = 0; t0 < a.rows; t0 += CT, buf ^= 1) {
+    if (t0 + CT < a.rows) load(t0 + CT);
+    const int nt = min(CT, a.rows - t0);
+    // the outputs of 8 tokens are summed over the lanes together, off the
+    // chain from token to token (rows_sum8: lane bits 0, 1, 2 hold token
+    // 4 b0 + 2 b1 + b2, each with wave_sum's bits)
+    for (int u0 = 0; u0 < nt; u0 += 8) {
+      double o[8];
+      if (u0 + 8 <= nt) {
+#pragma unroll
+        for (int u = 0; u < 8; u++) o[u] = token(buf, u0 + u);
+      } else {
+#pragma unroll
+        for (int u = 0; u < 8; u++) o[u] = u0 + u < nt ? token(buf, u0 + u) : 0.0;
+      }
+      int u;
+      rows_sum8(o, 32, u);
+      if (L < 8 && u0 + u < nt && j < a.dv)
+        a.y[(int64_t)(t0 + u0 + u) * vdw + (int64_t)head * a.dv + j] = (float)o[0];
+    }
+    // the other buffer was last read before the barrier that ended the chunk
+    // before this one
+    if (t0 + CT < a.rows) store(buf ^ 1);
+    __syncthreads();
+  }
+  if (j >= a.dv) return;
+#pragma unroll
+  for (int m = 0; m < NM; m++)
+#pragma unroll
+    for (int e = 0; e < 2; e++) {
+      const int i = 64 * m + 2 * L + e;
+      if (i < a.dk) col[i] = s[m][e];
+    }
+}
+extern "C" __global__ __launch_bounds__(256) void dn_rule_128(DnRuleArgs a) { dn_rule_chunks<2, 16>(a); }
+extern "C" __global__ __launch_bounds__(256) void dn_rule_256(DnRuleArgs a) { dn_rule_chunks<4, 8>(a); }
 
 struct DnNormArgs {
   float* x;        // [rows, cols]: the rule's output, normed and gated in place
