@@ -130,6 +130,9 @@ struct ihip_model {
   bool gemma = false;      // Gemma 4's settings: no fused one-row path
   // the widest heads of any layer, and the heads of the second rotary set
   int64_t max_qw = 0, max_kvw = 0, max_hd = 0, hd2 = 0;
+  // the rotary frequencies on the device (the second set's), and YaRN's scale
+  uint64_t rope_f = 0, rope_f2 = 0;
+  float rope_scale = 1.0f;
   // the host ranges of the uploaded weights: forgotten when the model goes,
   // as a model does in its destructor (backend.pas:151-158) - new host
   // tensors at a reused address must not meet the stale device copy
@@ -239,16 +242,23 @@ static void rotary(const ihip_model_desc& d, int64_t first, int64_t rows, float*
 // set over heads of hd2, 1 / theta2 ^ (2i / hd2) (each step rounded to
 // single) for the first rope2_pairs pairs, frequency 0 for the others; no
 // YaRN scale
-static void rotary2(const ihip_model_desc& d, int64_t hd2, int64_t first, int64_t rows, float* cs)
+static void inv_freq2(const ihip_model_desc& d, int64_t hd2, std::vector<float>& f)
 {
   const int64_t half = hd2 / 2;
   const double lt = std::log(d.rope2_theta);
-  std::vector<float> f(half, 0.f);
+  f.assign(half, 0.f);
   for (int64_t i = 0; i < half && i < d.rope2_pairs; i++) {
     float e = (float)((double)(2 * i) / (double)hd2);
     float p = (float)std::exp(lt * (double)e);
     f[i] = 1.0f / p;
   }
+}
+
+static void rotary2(const ihip_model_desc& d, int64_t hd2, int64_t first, int64_t rows, float* cs)
+{
+  const int64_t half = hd2 / 2;
+  std::vector<float> f;
+  inv_freq2(d, hd2, f);
   float* sn = cs + rows * half;
   for (int64_t r = 0; r < rows; r++)
     for (int64_t i = 0; i < half; i++) {
@@ -256,6 +266,23 @@ static void rotary2(const ihip_model_desc& d, int64_t hd2, int64_t first, int64_
       cs[r * half + i] = (float)std::cos((double)angle);
       sn[r * half + i] = (float)std::sin((double)angle);
     }
+}
+
+// the rotary rows of positions [first, first + rows) formed on the device from
+// the model's frequencies (rotary / rotary2): row r's cos at out + r stride,
+// its sin sin_at floats on
+static int rotary_dev(ihip_model* m, bool second, int64_t first, int64_t rows, uint64_t out, int64_t stride,
+                      int64_t sin_at)
+{
+  const int64_t half = second ? m->hd2 / 2 : rope_dims(m->d) / 2;
+  struct {
+    float* out;
+    const float* f;
+    float scale;
+    int32_t half, rows, first, stride, sin_at;
+  } a = {(float*)out, (const float*)(second ? m->rope_f2 : m->rope_f), second ? 1.0f : m->rope_scale,
+         (int32_t)half, (int32_t)rows, (int32_t)first, (int32_t)stride, (int32_t)sin_at};
+  return launch(m->c, "rotary_rows", dim3((unsigned)((rows * half + 255) / 256)), dim3(256), &a);
 }
 
 static int upw(ihip_model* m, const ihip_tensor& t, int64_t out, int64_t in, int64_t count,
@@ -1352,19 +1379,16 @@ static int chunk(ihip_mctx* s, const int32_t* ids, const float* embeds, int64_t 
   ihip_ctx* c = m->c;
   int rc0 = part_start(s, ids ? ids[0] : -1, first);
   if (rc0) return rc0;
-  std::vector<float> cs((size_t)n * d.head_dim), cs2((size_t)n * std::max<int64_t>(m->hd2, 1));
-  // declared after the host vectors, so destroyed before them: on every early
-  // return the queued copies from cs, cs2, ids and embeds have ended first
+  // on every early return the queued copies from ids and embeds have ended
+  // before the caller's memory goes
   struct StreamWait {
     hipStream_t st;
     ~StreamWait() { (void)hipStreamSynchronize(st); }
   } wait_copies{c->stream};
-  rotary(d, s->length, n, cs.data());
-  IHIP_CHECK(hipMemcpyHtoDAsync((hipDeviceptr_t)s->cs, cs.data(), cs.size() * 4, c->stream));
-  if (m->hd2) {
-    rotary2(d, m->hd2, s->length, n, cs2.data());
-    IHIP_CHECK(hipMemcpyHtoDAsync((hipDeviceptr_t)s->cs2, cs2.data(), cs2.size() * 4, c->stream));
-  }
+  const int64_t half = rope_dims(d) / 2;
+  if ((rc0 = rotary_dev(m, false, s->length, n, s->cs, half, n * half)) ||
+      (m->hd2 && (rc0 = rotary_dev(m, true, s->length, n, s->cs2, m->hd2 / 2, n * (m->hd2 / 2)))))
+    return rc0;
   int rc = s->length == 0 && m->recurrent ? reset_states(s) : 0;
   if (rc) return rc;
   if (ids) {
@@ -1462,15 +1486,10 @@ static int cs_table(ihip_mctx* s, int64_t upto)
   upto = std::min(upto, s->cs_cap);
   if (upto <= s->cs_rows) return 0;
   const int64_t n = upto - s->cs_rows;
-  std::vector<float> t((size_t)(n * rs), 0.f), t2((size_t)std::max<int64_t>(n * rs2, 1), 0.f);
-  for (int64_t r = 0; r < n; r++) {
-    rotary(m->d, s->cs_rows + r, 1, t.data() + r * rs);
-    if (rs2 > 0) rotary2(m->d, rs2, s->cs_rows + r, 1, t2.data() + r * rs2);
-  }
-  IHIP_CHECK(hipMemcpyHtoD((hipDeviceptr_t)(s->cs_tab + (uint64_t)s->cs_rows * rs * 4), t.data(), t.size() * 4));
-  if (rs2 > 0)
-    IHIP_CHECK(hipMemcpyHtoD((hipDeviceptr_t)(s->cs2_tab + (uint64_t)s->cs_rows * rs2 * 4), t2.data(),
-                             t2.size() * 4));
+  int rc = rotary_dev(m, false, s->cs_rows, n, s->cs_tab + (uint64_t)s->cs_rows * rs * 4, rs, rope_dims(m->d) / 2);
+  if (!rc && rs2 > 0)
+    rc = rotary_dev(m, true, s->cs_rows, n, s->cs2_tab + (uint64_t)s->cs_rows * rs2 * 4, rs2, rs2 / 2);
+  if (rc) return rc;
   s->cs_rows = upto;
   return 0;
 }
@@ -2238,6 +2257,22 @@ int ihip_model_create(ihip_ctx* c, const ihip_model_desc* desc, int mode, int kv
       all_gemm = all_gemm && gemm_runs(c, L.egd, mode) && gemm_runs(c, L.eud, mode) &&
                  gemm_runs(c, L.edd, mode);
   m->item_rows = all_gemm ? 64 : 8;
+  {
+    std::vector<float> f;
+    auto up = [&](uint64_t& dev) -> int {
+      void* p = nullptr;
+      IHIP_CHECK(hipMalloc(&p, f.size() * 4));
+      dev = (uint64_t)p;
+      IHIP_CHECK(hipMemcpyHtoD((hipDeviceptr_t)p, f.data(), f.size() * 4));
+      return 0;
+    };
+    inv_freq(d, f, m->rope_scale);
+    if ((rc = up(m->rope_f))) return bad(rc);
+    if (m->hd2) {
+      inv_freq2(d, m->hd2, f);
+      if ((rc = up(m->rope_f2))) return bad(rc);
+    }
+  }
   // the model's own context, its cache sized for max_tokens up front
   if ((rc = context_new(m, max_tokens, &m->def))) return bad(rc);
   m->def->is_default = true;
@@ -2252,6 +2287,8 @@ void ihip_model_destroy(ihip_model* m)
   for (ihip_mctx* s : m->contexts) context_free(s);
   m->contexts.clear();
   ihip_sampler_destroy(m->sampler);
+  if (m->rope_f) (void)hipFree((void*)m->rope_f);
+  if (m->rope_f2) (void)hipFree((void*)m->rope_f2);
   for (auto& u : m->uploaded) ihip_forget_weights(m->c, u.first, u.first + u.second);
   delete m;
 }

@@ -438,6 +438,36 @@ extern "C" __global__ __launch_bounds__(256) void softcap(SoftcapArgs a)
 }
 
 // ------------------------------------------------------------------ qkrope
+struct RotaryArgs {
+  float* out;
+  const float* f;  // [half] frequencies
+  float scale;     // YaRN's attention factor, 1: none
+  int32_t half, rows, first, stride, sin_at;  // row stride and sin offset of out, in floats
+};
+
+// cos and sin of positions first .. first + rows - 1, the host's steps
+// (TDecoderModel.Rotary, decoder.pas:2539-2561): the angle in single, cos and
+// sin of it in double rounded to single, then times the scale in single. On
+// the host the 1024 x 64 pairs of a prompt chunk were formed before its first
+// launch, with the GPU idle: a 1024-token pass of two Qwen3-30B-A3B layers 2979 ->
+// 2313 us with them formed here. One thread a pair; bound by the double cosine
+// and sine.
+extern "C" __global__ __launch_bounds__(256) void rotary_rows(RotaryArgs a)
+{
+  const int64_t n = (int64_t)blockIdx.x * 256 + threadIdx.x;
+  const int r = (int)(n / a.half), i = (int)(n % a.half);
+  if (r >= a.rows) return;
+  const float angle = a.f[i] * (float)(a.first + r);
+  float c = (float)cos((double)angle), s = (float)sin((double)angle);
+  if (a.scale != 1.0f) {
+    c = c * a.scale;
+    s = s * a.scale;
+  }
+  float* o = a.out + (int64_t)r * a.stride + i;
+  o[0] = c;
+  o[a.sin_at] = s;
+}
+
 struct RopeArgs {
   float* q;
   const float* k;
