@@ -450,7 +450,15 @@ int enqueue_linear(ihip_ctx* c, const LinearCall& k)
   if (k.items && k.item_rows > 8 && !gemm_q8)
     return fail(IHIP_E_ARG, "EnqueueLinear: items of more than 8 slots need the GEMM");
   const int min_rows = float_fmt(k.dtype) ? c->gemm_min_rows_float : c->gemm_min_rows;
-  if (batch && gemm_q8 && (k.items ? k.item_rows > 8 : k.rows >= min_rows)) {
+  // quantized weights, fewer rows than that: the 8-row launches below take
+  // about 5.5 us and 10 us per 10^6 (8 rows, output, group)s, the GEMM 5 us
+  // and 2 us per 1024 values of the sum, so the GEMM wins from about
+  // 6144 (8 rows, output)s whatever the sum's length (Q4_K, us, 8-row
+  // launches / GEMM: 16 rows of 2048 -> 6144 13.8 / 8.4, 16 of 1024 -> 3072
+  // 7.5 / 6.9, 48 of 3072 -> 1024 10.9 / 10.9, 32 of it 9.5 / 11.0, 64 of
+  // 2048 -> 512 8.2 / 9.2, 16 of 1024 -> 40000 20.4 / 11.3)
+  const bool few = q8 && c->gemm_few_rows && k.rows > 8 && (k.rows + 7) / 8 * k.out >= 6144;
+  if (batch && gemm_q8 && (k.items ? k.item_rows > 8 : k.rows >= min_rows || few)) {
     struct {
       const uint8_t* w;
       const uint8_t* xq;
@@ -515,7 +523,17 @@ int enqueue_linear(ihip_ctx* c, const LinearCall& k)
       g.xq = (const uint8_t*)c->scratch_planes;
       return launch(c, "gemm_mxfp4_f8", dim3(gx, gy), dim3(256), &g);
     }
-    return launch(c, gname, dim3(gx, gy), dim3(256), &g);
+    if (float_fmt(k.dtype)) return launch(c, gname, dim3(gx, gy), dim3(256), &g);
+    // blocks of 32 MT rows x 128 / KS outputs: from four 32 x 128 tiles a CU
+    // a K-quant takes 64 rows (its decode shared); with fewer than two a CU
+    // the waves of a block share the sum, in 2 parts, then in 4
+    const int64_t tiles32 = (k.items ? 2 * k.nitems : (k.rows + 31) / 32) * ((k.out + 127) / 128);
+    const bool wide = q8_kind(k.dtype) == 1 && (k.items || tiles32 >= 4 * (int64_t)c->cus);
+    const int ks = k.items || tiles32 >= 2 * (int64_t)c->cus ? 1 : 4 * tiles32 >= 3 * (int64_t)c->cus ? 2 : 4;
+    snprintf(gname, sizeof gname, "gemm_%s_m%dk%d", fmt_name(k.dtype), wide ? 2 : 1, ks);
+    const unsigned by = (unsigned)(k.items ? (wide ? 1 : 2) * k.nitems : (k.rows + (wide ? 63 : 31)) / (wide ? 64 : 32));
+    const int64_t bn = 128 / ks;
+    return launch(c, gname, dim3((unsigned)((k.out + bn - 1) / bn), by), dim3(256), &g);
   }
   if (k.nw && (batch || k.in > 4096 || xq))
     return fail(IHIP_E_ARG, "EnqueueLinear: the fused rmsnorm takes one float row of at most 4096");

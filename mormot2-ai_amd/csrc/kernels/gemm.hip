@@ -8,17 +8,28 @@
 // GEMV of linear.hip (group_q8, group_q8k, superblock_q8k); only the order of
 // the double sum over groups differs (here: group order).
 //
-// Mapping to CDNA4: a block of 4 waves owns 64 rows x 64 outputs, each wave
-// 32 x 32. Per 32-value group a wave runs v_mfma_i32_32x32x32_i8 with A = the
-// activation codes of its 32 rows and B = the weight codes of its 32
-// outputs, widened to int8 (centred for Q4_0/Q5_0/Q6_K, the e2m1 table for
-// MXFP4): the exact int32 group dot products, 16 per lane. The lanes then
-// apply the scales in double: a lane owns one output (its scales are
-// per-lane registers) and 16 rows (their activation scales and code sums are
-// staged in LDS per 8 groups). Q6_K's 16-value sub-blocks are two
-// v_mfma_i32_32x32x16_i8, lane half h feeding values 8h..8h+7 of each
-// sub-block: with the group's nibble order (byte j: value j, value j + 16)
-// both come from bytes 8h..8h+7 of the 16-byte group.
+// Mapping to CDNA4: a wave owns one or two tiles of 32 rows x 32 outputs. Per
+// 32-value group it runs v_mfma_i32_32x32x32_i8 with A = the activation codes
+// of a tile's rows and B = the weight codes of its outputs, widened to int8
+// (centred for Q4_0/Q5_0/Q6_K, the e2m1 table for MXFP4): the exact int32
+// group dot products, 16 per lane. The scales follow: a lane owns one output
+// and 16 rows. For the formats of 32 values the products dw dx of all its
+// outputs come from one outer-product MFMA (v_mfma_f32_32x32x16_f16 with one
+// k: two halves, the product exact in single), where reading 16 row scales a
+// group from LDS cost more than the group's arithmetic; then one fused
+// multiply-add in double per output. K-quants multiply the group sums by their
+// integer sub-scales and form one term per super-block; Q4_K's minimum sum is
+// one f16 MFMA a super-block over the code sums split 64 hi + lo. Q6_K's
+// 16-value sub-blocks are two v_mfma_i32_32x32x16_i8, lane half h feeding
+// values 8h..8h+7 of each: with the group's nibble order (byte j: value j,
+// value j + 16) both come from bytes 8h..8h+7 of the 16-byte group.
+//
+// Bound by the vector unit and the chain LDS -> widening -> MFMA -> terms of
+// a group, which two or three waves a SIMD cover; 41 (Q4_K) to 60 vector
+// instructions per tile and group. Measured against the 64 x 64 tiles with
+// row scales in LDS that this replaces, us: Q4_K 512 rows 2048 -> 6144
+// 47.5 -> 31.9 (403 TOP/s), 1024 rows 2048 -> 4096 37.4 (459), Q6_K 512 rows
+// 60 -> 51, Q8_0 301 rows 3072 -> 1024 34.7 -> 17.5 (the sum over 4 waves).
 //
 // Operand layout of both MFMAs (probed on gfx950): A lane l = row l % 32,
 // B lane l = column l % 32, 16 (8) k values each, the k order free but the
@@ -30,6 +41,8 @@ namespace ihip {
 
 typedef int v4i __attribute__((ext_vector_type(4)));
 typedef int v16i __attribute__((ext_vector_type(16)));
+typedef float v16f_t __attribute__((ext_vector_type(16)));
+typedef _Float16 v8h_t __attribute__((ext_vector_type(8)));
 
 struct GemmArgs {
   const uint8_t* w;   // matrix, or expert 0 with items
@@ -51,27 +64,16 @@ struct GemmArgs {
   int32_t ksplit, klen;
 };
 
-constexpr int GBM = 64, GBN = 64, GKC = 8;  // tile rows, outputs, groups per chunk
+constexpr int GBM = 64, GBN = 64;  // tile rows and outputs (float weights, f8f6f4)
+constexpr int GKC = 8;             // groups per chunk: 256 values, a K-quant super-block
 
-// the weight codes of lane half h (values 8h..8h+7 and 16+8h..16+8h+7 of the
-// group) as 16 int8 in the Q8 arithmetic's value (centred where the format
-// has an offset the CPU subtracts through the activation sum)
+// the 16 codes of code dwords 0 and 1 (values 0..7 of the low half of a
+// group's bytes, then of the high) as int8 in the Q8 arithmetic's value
+// (centred where the format has an offset the CPU subtracts through the
+// activation sum)
 template <int F>
-__device__ __forceinline__ v4i b_operand(const Raw& r, int h)
+__device__ __forceinline__ v4i widen(const Raw& v)
 {
-  // the lane half's view of the group: code dwords 2h and 2h + 1 moved to
-  // dwords 0 and 1, chosen by masks (values, never an index into registers)
-  const uint32_t m = 0u - (uint32_t)h;
-  Raw v = r;
-  v.q0.x = (r.q0.x & ~m) | (r.q0.z & m);
-  v.q0.y = (r.q0.y & ~m) | (r.q0.w & m);
-  v.q1.x = (r.q1.x & ~m) | (r.q1.z & m);
-  v.q1.y = (r.q1.y & ~m) | (r.q1.w & m);
-  if constexpr (F == DT_Q5_0 || F == DT_Q5_1) v.b = r.b >> (8 * h);  // 4 bits per code dword
-  if constexpr (F == DT_Q6_K) {  // 2 bits per code dword
-    v.b = r.b >> (4 * h);
-    v.c = r.c >> (4 * h);
-  }
   uint32_t c[4] = {code_bytes<F>(v, 0, 0), code_bytes<F>(v, 1, 0), code_bytes<F>(v, 0, 1),
                    code_bytes<F>(v, 1, 1)};
 #pragma unroll
@@ -90,6 +92,26 @@ __device__ __forceinline__ v4i b_operand(const Raw& r, int h)
     c[k] = t;
   }
   return v4i{(int)c[0], (int)c[1], (int)c[2], (int)c[3]};
+}
+
+// widen() of lane half h (values 8h..8h+7 and 16+8h..16+8h+7 of the group)
+template <int F>
+__device__ __forceinline__ v4i b_operand(const Raw& r, int h)
+{
+  // the lane half's view of the group: code dwords 2h and 2h + 1 moved to
+  // dwords 0 and 1, chosen by masks (values, never an index into registers)
+  const uint32_t m = 0u - (uint32_t)h;
+  Raw v = r;
+  v.q0.x = (r.q0.x & ~m) | (r.q0.z & m);
+  v.q0.y = (r.q0.y & ~m) | (r.q0.w & m);
+  v.q1.x = (r.q1.x & ~m) | (r.q1.z & m);
+  v.q1.y = (r.q1.y & ~m) | (r.q1.w & m);
+  if constexpr (F == DT_Q5_0 || F == DT_Q5_1) v.b = r.b >> (8 * h);  // 4 bits per code dword
+  if constexpr (F == DT_Q6_K) {  // 2 bits per code dword
+    v.b = r.b >> (4 * h);
+    v.c = r.c >> (4 * h);
+  }
+  return widen<F>(v);
 }
 
 // does the format need the activation code sum of a group (through the
@@ -140,72 +162,7 @@ __device__ __forceinline__ Raw raw_get(const uint32_t* d, int stride)
   return r;
 }
 
-// A chunk of GKC groups of a block's tile, loaded cooperatively with
-// coalesced accesses (each group of 8 lanes reads 8 consecutive groups of one
-// weight row; each 4 lanes one activation row's 256 code bytes) into
-// registers, then stored to LDS: the operands reach the lanes that feed
-// the MFMAs from LDS, never as 32 scattered rows per load instruction.
-struct ChunkRegs {
-  Raw wr[2];      // weight groups: column t / 8 (+ 32), group t % 8
-  v4u32 xc[4];    // activation codes: row t / 4, groups 2 (t % 4) and 2 (t % 4) + 1
-  float dx[2];    // and their scales
-  v4u32 xp[4];    // F8: the second half of the groups' 64-byte e4m3 planes
-};
-
-
-
-template <int F>
-__device__ __forceinline__ void chunk_load(const GemmArgs& a, const uint8_t* wb, const Regions& rg,
-                                           int col0, const int* sxr, int64_t xstride, int G, int gc,
-                                           ChunkRegs& cr)
-{
-  const int t = threadIdx.x;
-#pragma unroll
-  for (int p = 0; p < 2; p++) {
-    const int64_t o = min(col0 + (t >> 3) + 32 * p, a.out - 1);
-    load_group<F>(wb, rg, o, G, min(gc + (t & 7), G - 1), a.in, cr.wr[p]);
-  }
-  const uint8_t* xr = a.xq + (int64_t)sxr[t >> 2] * xstride;
-#pragma unroll
-  for (int k = 0; k < 2; k++) {
-    const int g = min(gc + 2 * (t & 3) + k, G - 1);
-    const v4u32* q = (const v4u32*)(xr + (int64_t)g * 32);
-    cr.xc[2 * k] = q[0];
-    cr.xc[2 * k + 1] = q[1];
-    cr.dx[k] = ((const float*)(xr + a.in))[g];
-  }
-}
-
-constexpr int GSW = GKC * raw_dwords<DT_Q8_0>() + 1;  // LDS dwords per weight column (odd)
-constexpr int GSA = GKC * 8 + 2;                     // LDS dwords per activation row
-
-template <int F>
-__device__ __forceinline__ void chunk_store(const ChunkRegs& cr, uint32_t* sw, uint32_t* sa, double* sdx,
-                                            int* sbs)
-{
-  const int t = threadIdx.x;
-  constexpr int WS = GKC * raw_dwords<F>() + 1;  // this format's column stride
-#pragma unroll
-  for (int p = 0; p < 2; p++) raw_put<F>(sw + ((t >> 3) + 32 * p) * WS + (t & 7), GKC, cr.wr[p]);
-  const int row = t >> 2;
-#pragma unroll
-  for (int k = 0; k < 2; k++) {
-    const int j = 2 * (t & 3) + k;
-    uint32_t* d = sa + row * GSA + j * 8;
-    *(v4u32*)d = cr.xc[2 * k];
-    *(v4u32*)(d + 4) = cr.xc[2 * k + 1];
-    sdx[j * GBM + row] = (double)cr.dx[k];  // widened once here, not per output
-    if constexpr (needs_xsum(F) && F != DT_Q4_K) {  // (Q4_K: the m_j sums on the matrix cores)
-      const v4u32 u0 = cr.xc[2 * k], u1 = cr.xc[2 * k + 1];
-      int sm = 0;
-      sm = sdot4((int)u0.x, 0x01010101, sm); sm = sdot4((int)u0.y, 0x01010101, sm);
-      sm = sdot4((int)u0.z, 0x01010101, sm); sm = sdot4((int)u0.w, 0x01010101, sm);
-      sm = sdot4((int)u1.x, 0x01010101, sm); sm = sdot4((int)u1.y, 0x01010101, sm);
-      sm = sdot4((int)u1.z, 0x01010101, sm); sm = sdot4((int)u1.w, 0x01010101, sm);
-      sbs[j * GBM + row] = sm;
-    }
-  }
-}
+constexpr int G8A = 8 * 8 + 2;  // gemm8: LDS dwords per activation row
 
 // ------------------------------------------- MXFP4 on the scaled f8f6f4 MFMA
 // v_mfma_scale_f32_32x32x64_f8f6f4 with B the group's e2m1 codes as they are
@@ -227,7 +184,15 @@ __device__ __forceinline__ void chunk_store(const ChunkRegs& cr, uint32_t* sw, u
 // 0, 1 the 32 bytes e4m3(16 hi[v(16h + j)]) j < 16, e4m3(lo[v(16h + j)]) j
 // < 16 - lane half h reads bytes 32h..32h+31 of the group.
 typedef int v8i_t __attribute__((ext_vector_type(8)));
-typedef float v16f_t __attribute__((ext_vector_type(16)));
+
+// a chunk of GKC groups of the tile in registers, from coalesced loads
+struct ChunkRegs {
+  Raw wr[2];      // weight groups: column t / 8 (+ 32), group t % 8
+  v4u32 xc[4];    // the first half of the planes: row t / 4, groups 2 (t % 4) and 2 (t % 4) + 1
+  float dx[2];    // and their scales
+  v4u32 xp[4];    // the second half
+};
+constexpr int GSW = GKC * raw_dwords<DT_Q8_0>() + 1;  // LDS dwords per weight column (odd)
 
 // e4m3 of an integer in [-8, 8] (times 16 when x16: the exponent + 4)
 __device__ __forceinline__ uint32_t e4m3_small(int v, bool x16)
@@ -423,198 +388,440 @@ __device__ __forceinline__ void f8_planes(const PlanesArgs& a)
   ((float*)(dst + (int64_t)G * 64))[gi] = ((const float*)(src + a.in))[gi];
 }
 
+// Block shapes. A block has 4 waves; a wave owns MT tiles of 32 rows x 32
+// outputs and every KS-th chunk of the sum, the 4 / KS waves across make
+// 32 MT rows x 128 / KS outputs, and the KS partial sums of an output meet in
+// LDS at the end.
+constexpr int GSA = 68;  // LDS dwords of an activation row's chunk (64 and a 16-byte shift of banks)
+
+// code dwords of a group, and the dwords beside them (scale, high bits)
 template <int F>
-__device__ __forceinline__ void gemm(const GemmArgs& a)
+constexpr int code_dwords() { return F == DT_Q8_0 ? 8 : 4; }
+template <int F>
+constexpr int side_dwords()
 {
-  // one chunk's operands: weight groups by column, activation codes by row,
-  // the rows' scales and code sums
-  __shared__ uint32_t sw_[GBN * GSW];
-  __shared__ __align__(16) uint32_t sa_[GBM * GSA];
-  __shared__ __align__(16) double sdx_[GKC * GBM];
-  __shared__ int sbs_[needs_xsum(F) ? GKC * GBM : 1];
-  __shared__ int sxr[GBM], syr[GBM];
-  const int t = threadIdx.x, l = t & 63, w = t >> 6, h = l >> 5;
-  const int wm = w & 1, wn = w >> 1;
+  return F == DT_Q4_K ? 0 : F == DT_Q6_K ? 3 : (F == DT_Q5_0 || F == DT_Q5_1) ? 2 : 1;
+}
+constexpr bool kquant(int F) { return F == DT_Q4_K || F == DT_Q6_K; }
+// LDS dwords of a weight column's codes of a chunk: the 32 columns of a wave
+// read 8 (Q8_0: 16) bytes each at one group, 2 (4) dwords a column apart
+template <int F>
+constexpr int col_dwords() { return F == DT_Q8_0 ? 68 : 34; }
+
+// LDS of a block, in dwords: the regions of one step (4 wave slots of weights,
+// KS chunks of activation rows), reused by the partial sums
+template <int F, int MT, int KS>
+struct GemmLds {
+  static constexpr int A = 0;                                    // codes [KS][32 MT][GSA]
+  static constexpr int B = A + KS * 32 * MT * GSA;               // codes [4][32][col_dwords]
+  static constexpr int X = B + 128 * col_dwords<F>();            // side dwords [.][GKC][128]
+  static constexpr int H = X + side_dwords<F>() * GKC * 128;     // K-quants: header [128][4]
+  static constexpr int D = H + (F == DT_Q4_K ? 512 : F == DT_Q6_K ? 128 : 0);
+  // K-quants: a double per row; else the scale's half bits per (group, row)
+  static constexpr int S = D + (kquant(F) ? KS * 32 * MT * 2 : KS * GKC * 32 * MT);
+  // Q4_K: the code sums as halves [KS][32 MT][16]; Q5_1: dx times the sum, doubles
+  static constexpr int END = S + (F == DT_Q4_K ? KS * 32 * MT * 8 : F == DT_Q5_1 ? KS * GKC * 32 * MT * 2 : 0);
+  static constexpr int RED = (KS - 1) * (4 / KS) * MT * 2048;    // partial sums, doubles
+  static constexpr int DWORDS = END > RED ? END : RED;
+};
+
+// a step's operands in registers, from coalesced loads (each 8 lanes read 8
+// consecutive groups of a weight row, or a row's 256 activation codes)
+template <int F, int MT, int KS>
+struct StepRegs {
+  Raw wr[4];               // slot p: column t / 8 of wave slot p, group t % 8
+  v4u32 xc[KS * MT][2];    // rows t / 8 + 32 mt, group t % 8 of chunk ks
+  float dx[KS * MT];
+};
+
+template <int F, int MT, int KS>
+__device__ __forceinline__ void step_load(const GemmArgs& a, const uint8_t* wb, const Regions& rg, int col0,
+                                          const int* sxr, int64_t xstride, int G, int g0,
+                                          StepRegs<F, MT, KS>& r)
+{
+  const int t = threadIdx.x;
+  // groups past the last read the last one again; their scales are zero, so
+  // their terms are
+#pragma unroll
+  for (int p = 0; p < 4; p++) {
+    const int64_t o = min(col0 + 32 * (p / KS) + (t >> 3), a.out - 1);
+    const int g = g0 + GKC * (p % KS) + (t & 7);
+    load_group<F, false, true>(wb, rg, o, G, min(g, G - 1), a.in, r.wr[p]);
+    if (!kquant(F) && g >= G) r.wr[p].a = 0;
+  }
+#pragma unroll
+  for (int q = 0; q < KS * MT; q++) {
+    const int g = g0 + GKC * (q / MT) + (t & 7), gl = min(g, G - 1);
+    const uint8_t* xr = a.xq + (int64_t)sxr[32 * (q % MT) + (t >> 3)] * xstride;
+    const v4u32* c = (const v4u32*)(xr + (int64_t)gl * 32);
+    r.xc[q][0] = c[0];
+    r.xc[q][1] = c[1];
+    r.dx[q] = ((const float*)(xr + a.in))[gl];
+    if (!kquant(F) && g >= G) r.dx[q] = 0.0f;
+  }
+}
+
+__device__ __forceinline__ uint32_t half_bits(float v)
+{
+  return (uint32_t)__builtin_bit_cast(uint16_t, (_Float16)v);
+}
+
+template <int F, int MT, int KS>
+__device__ __forceinline__ void step_store(const StepRegs<F, MT, KS>& r, uint32_t* lds)
+{
+  using L = GemmLds<F, MT, KS>;
+  const int t = threadIdx.x, g = t & 7;
+#pragma unroll
+  for (int p = 0; p < 4; p++) {
+    const int col = 32 * p + (t >> 3);
+    uint32_t* d = lds + L::B + col * col_dwords<F>() + g * code_dwords<F>();
+    const Raw& w = r.wr[p];
+    if constexpr (F == DT_Q8_0) {
+      *(uint4*)d = w.q0;
+      *(uint4*)(d + 4) = w.q1;
+    } else {
+      *(uint2*)d = make_uint2(w.q0.x, w.q0.y);
+      *(uint2*)(d + 2) = make_uint2(w.q0.z, w.q0.w);
+    }
+    uint32_t* x = lds + L::X + g * 128 + col;
+    if constexpr (F == DT_Q4_K) {
+      if (g < 4) lds[L::H + 4 * col + g] = w.q1.x;  // (QH: dword t % 4 of the header)
+    } else if constexpr (F == DT_Q6_K) {
+      x[0] = w.a;
+      x[GKC * 128] = w.b;
+      x[2 * GKC * 128] = w.c;
+      if (g == 0) lds[L::H + col] = w.d;
+    } else {
+      x[0] = F == DT_MXFP4 ? half_bits((float)mxfp4_q8_scale(w.a)) : w.a;
+      if constexpr (F == DT_Q5_0 || F == DT_Q5_1) x[GKC * 128] = w.b;
+    }
+  }
+#pragma unroll
+  for (int q = 0; q < KS * MT; q++) {
+    const int row = 32 * (q % MT) + (t >> 3), kr = (q / MT) * 32 * MT + row;
+    const v4u32 u0 = r.xc[q][0], u1 = r.xc[q][1];
+    uint32_t* d = lds + L::A + kr * GSA + g * 8;
+    // lane half h of the MFMA reads 16 bytes: the values its weight bytes hold
+    if constexpr (F == DT_Q8_0) {
+      *(v4u32*)d = u0;
+      *(v4u32*)(d + 4) = u1;
+    } else {
+      *(v4u32*)d = v4u32{u0.x, u0.y, u1.x, u1.y};
+      *(v4u32*)(d + 4) = v4u32{u0.z, u0.w, u1.z, u1.w};
+    }
+    if constexpr (kquant(F)) {
+      if (g == 0) ((double*)(lds + L::D))[kr] = (double)r.dx[q];
+    } else {
+      lds[L::D + (q / MT) * GKC * 32 * MT + g * 32 * MT + row] = half_bits(r.dx[q]);
+    }
+    if constexpr (F == DT_Q4_K || F == DT_Q5_1) {
+      int sm = 0;
+      sm = sdot4((int)u0.x, 0x01010101, sm); sm = sdot4((int)u0.y, 0x01010101, sm);
+      sm = sdot4((int)u0.z, 0x01010101, sm); sm = sdot4((int)u0.w, 0x01010101, sm);
+      sm = sdot4((int)u1.x, 0x01010101, sm); sm = sdot4((int)u1.y, 0x01010101, sm);
+      sm = sdot4((int)u1.z, 0x01010101, sm); sm = sdot4((int)u1.w, 0x01010101, sm);
+      if constexpr (F == DT_Q4_K) {
+        // sum = 64 hi + lo, each exact in half: lo of the 8 groups, then hi
+        uint16_t* s = (uint16_t*)(lds + L::S) + kr * 16 + g;
+        s[0] = (uint16_t)half_bits((float)(sm & 63));
+        s[8] = (uint16_t)half_bits((float)(sm >> 6));
+      } else {
+        ((double*)(lds + L::S))[(q / MT) * GKC * 32 * MT + g * 32 * MT + row] = (double)r.dx[q] * (double)sm;
+      }
+    }
+  }
+}
+
+// four bytes below 64 as two pairs of halves (1024 + b as bits, then - 1024)
+__device__ __forceinline__ v8h_t bytes_half8(uint32_t b0, uint32_t b1, _Float16 times)
+{
+  typedef _Float16 v2h __attribute__((ext_vector_type(2)));
+  const v2h off = {(_Float16)-1024.0f, (_Float16)-1024.0f}, mul = {times, times};
+  v8h_t v;
+#pragma unroll
+  for (int k = 0; k < 4; k++) {
+    const uint32_t w = __builtin_amdgcn_perm(0x64646464u, k < 2 ? b0 : b1, (k & 1) ? 0x04030402u : 0x04010400u);
+    const v2h h = (__builtin_bit_cast(v2h, w) + off) * mul;
+    v[2 * k] = h.x;
+    v[2 * k + 1] = h.y;
+  }
+  return v;
+}
+
+// a value the compiler may not reassociate through: it would hold the products
+// of a whole super-block to sum them in another order, and spill
+__device__ __forceinline__ int keep(int v)
+{
+  __asm__("" : "+v"(v));
+  return v;
+}
+
+template <int F, int MT, int KS>
+__device__ __forceinline__ void gemm_tiles(const GemmArgs& a, const uint8_t* wb, const float* bias, int nrows,
+                                           const int* sxr, const int* syr, uint32_t* lds)
+{
+  using L = GemmLds<F, MT, KS>;
+  const int t = threadIdx.x, l = t & 63, w = t >> 6, h = l >> 5, c32 = l & 31;
+  const int wn = w / KS, ks = w % KS;
   const int G = a.in >> 5;
   const int64_t xstride = (int64_t)a.in + 4 * (int64_t)G;
+  const Regions rg = regions(F, a.out, a.in);
+  const int col0 = blockIdx.x * (128 / KS);
+  // this lane's weight column and activation rows in LDS
+  const int col = 32 * w + c32;
+  const uint32_t* myb = lds + L::B + col * col_dwords<F>() + h * (code_dwords<F>() / 2);
+  const uint32_t* mya = lds + L::A + (ks * 32 * MT + c32) * GSA + 4 * h;
+  const uint32_t* myx = lds + L::X + col;
+  const uint32_t lowhalf = h ? 0u : 0xffffu;
+
+  double acc[MT][16];
+  int isum[MT][16];
+#pragma unroll
+  for (int m = 0; m < MT; m++)
+#pragma unroll
+    for (int i = 0; i < 16; i++) {
+      acc[m][i] = 0.0;
+      isum[m][i] = 0;
+    }
+  const v16i zi = {};
+  const v16f_t zf = {};
+
+  // the operands of a group read from LDS
+  struct Ops {
+    uint2 q;         // this lane half's code bytes
+    v4u32 q16;       // (Q8_0)
+    uint32_t x, b, c;  // scale and high bits
+    v4u32 xa[MT];    // activation codes
+    uint32_t dx[MT];   // the scale of the lane's row, as half bits
+  };
+  struct Sums {
+    v16i s, s2;   // group sums (Q6_K: of its two sub-blocks)
+    v16f_t p;     // dw dx of every output (block formats of 32 values)
+  };
+  auto read = [&](int j) __attribute__((always_inline)) -> Ops {
+    Ops r = {};
+    if constexpr (F == DT_Q8_0) r.q16 = *(const v4u32*)(myb + j * 8);
+    else r.q = *(const uint2*)(myb + j * 4);
+    if constexpr (F != DT_Q4_K) r.x = myx[j * 128];
+    if constexpr (side_dwords<F>() > 1) r.b = myx[(GKC + j) * 128];
+    if constexpr (side_dwords<F>() > 2) r.c = myx[(2 * GKC + j) * 128];
+#pragma unroll
+    for (int m = 0; m < MT; m++) {
+      r.xa[m] = *(const v4u32*)(mya + m * 32 * GSA + j * 8);
+      if constexpr (!kquant(F)) r.dx[m] = lds[L::D + (ks * GKC + j) * 32 * MT + 32 * m + c32];
+    }
+    return r;
+  };
+  // the group's weight codes as int8 in the lanes' order
+  auto codes = [&](const Ops& r) __attribute__((always_inline)) -> v4i {
+    if constexpr (F == DT_Q8_0) {
+      return __builtin_bit_cast(v4i, r.q16);
+    } else {
+      Raw v{};
+      v.q0.x = r.q.x;
+      v.q0.y = r.q.y;
+      if constexpr (F == DT_Q5_0 || F == DT_Q5_1) v.b = r.b >> (8 * h);
+      if constexpr (F == DT_Q6_K) {
+        v.b = r.b >> (4 * h);
+        v.c = r.c >> (4 * h);
+      }
+      return widen<F>(v);
+    }
+  };
+  auto multiply = [&](const Ops& g, int m, const v4i& b) __attribute__((always_inline)) -> Sums {
+    const v4i x = __builtin_bit_cast(v4i, g.xa[m]);
+    Sums r;
+    if constexpr (F == DT_Q6_K) {
+      r.s = __builtin_amdgcn_mfma_i32_32x32x16_i8((long)(((uint64_t)(uint32_t)x.y << 32) | (uint32_t)x.x),
+                                                  (long)(((uint64_t)(uint32_t)b.y << 32) | (uint32_t)b.x), zi, 0, 0, 0);
+      r.s2 = __builtin_amdgcn_mfma_i32_32x32x16_i8((long)(((uint64_t)(uint32_t)x.w << 32) | (uint32_t)x.z),
+                                                   (long)(((uint64_t)(uint32_t)b.w << 32) | (uint32_t)b.z), zi, 0, 0, 0);
+    } else {
+      r.s = __builtin_amdgcn_mfma_i32_32x32x32_i8(x, b, zi, 0, 0, 0);
+    }
+    if constexpr (!kquant(F)) {
+      // dw dx of the 32 x 32 outputs as one outer product (k = 0 alone): both
+      // halves, the product exact in single
+      const v4u32 av = {g.dx[m] & lowhalf, 0, 0, 0}, bv = {g.x & lowhalf, 0, 0, 0};
+      r.p = __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(v8h_t, av), __builtin_bit_cast(v8h_t, bv), zf,
+                                                   0, 0, 0);
+    }
+    return r;
+  };
+  // Q4_K: the scales of groups 0..3 and 4..7 of the super-block, as bytes
+  uint32_t sc0 = 0, sc1 = 0, hd0 = 0;
+  // the terms of group j: K-quants into the super-block's integer sum, else
+  // into the double sum (s dw dx is exact, one rounding per group)
+  auto terms = [&](int j, int m, const Sums& r, uint32_t x) __attribute__((always_inline)) {
+    if constexpr (F == DT_Q4_K) {
+      const int sc = (int)(((j & 4) ? sc1 : sc0) >> (8 * (j & 3))) & 255;
+#pragma unroll
+      for (int i = 0; i < 16; i++) isum[m][i] = keep(isum[m][i] + __mul24(sc, r.s[i]));  // |sums| < 2^16, sc < 64
+    } else if constexpr (F == DT_Q6_K) {
+      const int sa = (int)(int8_t)(x & 255u), sb = (int)(int8_t)(x >> 8);
+#pragma unroll
+      for (int i = 0; i < 16; i++)
+        isum[m][i] = keep(keep(isum[m][i] + __mul24(sa, r.s[i])) + __mul24(sb, r.s2[i]));
+    } else {
+#pragma unroll
+      for (int i = 0; i < 16; i++) acc[m][i] = __builtin_fma((double)r.s[i], (double)r.p[i], acc[m][i]);
+      if constexpr (F == DT_Q5_1) {
+        const double m51 = half_to_float(x >> 16);
+        const double* xs = (const double*)(lds + L::S) + (ks * GKC + j) * 32 * MT + 32 * m + 4 * h;
+#pragma unroll
+        for (int i = 0; i < 16; i++) acc[m][i] = __builtin_fma(m51, xs[8 * (i >> 2) + (i & 3)], acc[m][i]);
+      }
+    }
+  };
+
+  StepRegs<F, MT, KS> r;
+  const int nch = (G + GKC - 1) / GKC, nst = (nch + KS - 1) / KS;
+  step_load<F, MT, KS>(a, wb, rg, col0, sxr, xstride, G, 0, r);
+  step_store<F, MT, KS>(r, lds);
+  step_load<F, MT, KS>(a, wb, rg, col0, sxr, xstride, G, GKC * KS, r);
+  __syncthreads();
+  for (int c = 0; c < nst; c++) {
+    const int ng = min(GKC, G - (c * KS + ks) * GKC);  // groups of this wave's chunk
+    if constexpr (F == DT_Q4_K) {
+      const uint4 hd = *(const uint4*)(lds + L::H + 4 * col);  // (scale_min_k4)
+      sc0 = hd.y & 0x3f3f3f3fu;
+      sc1 = (hd.w & 0x0f0f0f0fu) | ((hd.y >> 2) & 0x30303030u);
+      hd0 = hd.x;
+    }
+    // (a chunk past the last: no terms; groups past the last in a chunk have
+    // zero scales)
+    if (ng > 0) {
+      Ops g = read(0);
+#pragma unroll
+      for (int j = 0; j < GKC; j++) {
+        const v4i b = codes(g);
+        Sums s[MT];
+#pragma unroll
+        for (int m = 0; m < MT; m++) s[m] = multiply(g, m, b);
+        const uint32_t x = g.x;
+        // the next group's LDS reads are under way while the terms are formed
+        if (j + 1 < GKC) g = read(j + 1);
+#pragma unroll
+        for (int m = 0; m < MT; m++) {
+          terms(j, m, s[m], x);
+          // (free to move them further, the scheduler would spill)
+          __builtin_amdgcn_sched_barrier(0);
+        }
+      }
+    }
+    if constexpr (kquant(F)) {
+      // the super-block's term (rows hold whole ones): d dx isum, Q4_K
+      // - dmin dx sum_j m_j bsum_j, the sum exact from one f16 MFMA over the
+      // halves of the code sums (lane half 0: lo m_j, 1: hi 64 m_j)
+      if (ng > 0) {
+        double d, dm = 0;
+        v8h_t bm;
+        if constexpr (F == DT_Q4_K) {
+          const uint4 hd = *(const uint4*)(lds + L::H + 4 * col);
+          d = half_to_float(hd0 & 0xffffu);
+          dm = -(double)half_to_float(hd0 >> 16);
+          bm = bytes_half8(hd.z & 0x3f3f3f3fu, ((hd.w >> 4) & 0x0f0f0f0fu) | ((hd.z >> 2) & 0x30303030u),
+                           (_Float16)(h ? 64.0f : 1.0f));
+        } else {
+          d = half_to_float(lds[L::H + col]);
+        }
+#pragma unroll
+        for (int m = 0; m < MT; m++) {
+          const double* xs = (const double*)(lds + L::D) + ks * 32 * MT + 32 * m + 4 * h;
+          v16f_t cm;
+          if constexpr (F == DT_Q4_K) {
+            const v8h_t am = *(const v8h_t*)(lds + L::S + (ks * 32 * MT + 32 * m + c32) * 8 + 4 * h);
+            cm = __builtin_amdgcn_mfma_f32_32x32x16_f16(am, bm, zf, 0, 0, 0);
+          }
+#pragma unroll
+          for (int i = 0; i < 16; i++) {
+            double v = d * (double)isum[m][i];
+            if constexpr (F == DT_Q4_K) v = __builtin_fma(dm, (double)cm[i], v);
+            acc[m][i] = __builtin_fma(xs[8 * (i >> 2) + (i & 3)], v, acc[m][i]);
+            isum[m][i] = 0;
+          }
+        }
+      }
+    }
+    __syncthreads();  // the step's LDS reads are done
+    if (c + 1 < nst) {
+      step_store<F, MT, KS>(r, lds);
+      if (c + 2 < nst) step_load<F, MT, KS>(a, wb, rg, col0, sxr, xstride, G, (c + 2) * GKC * KS, r);
+      __syncthreads();
+    }
+  }
+  if constexpr (KS > 1) {
+    // the partial sums of wave ks > 0 through LDS to wave ks = 0 of the column
+    double* red = (double*)lds;
+    if (ks > 0) {
+#pragma unroll
+      for (int m = 0; m < MT; m++)
+#pragma unroll
+        for (int i = 0; i < 16; i++) red[(((wn * (KS - 1) + ks - 1) * MT + m) * 16 + i) * 64 + l] = acc[m][i];
+    }
+    __syncthreads();
+    if (ks > 0) return;
+#pragma unroll
+    for (int q = 0; q < KS - 1; q++)
+#pragma unroll
+      for (int m = 0; m < MT; m++)
+#pragma unroll
+        for (int i = 0; i < 16; i++) acc[m][i] += red[(((wn * (KS - 1) + q) * MT + m) * 16 + i) * 64 + l];
+  }
+  const int o = col0 + 32 * wn + c32;
+  if (o >= a.out) return;
+  const double b = bias ? (double)bias[o] : 0.0;
+#pragma unroll
+  for (int m = 0; m < MT; m++)
+#pragma unroll
+    for (int i = 0; i < 16; i++) {
+      const int rt = 32 * m + 8 * (i >> 2) + 4 * h + (i & 3);
+      if (rt < nrows) {
+        double v = acc[m][i];
+        if (bias) v = b + v;
+        a.y[(int64_t)syr[rt] * a.out + o] = (float)v;
+      }
+    }
+}
+
+template <int F, int MT, int KS>
+__device__ __forceinline__ void gemm(const GemmArgs& a)
+{
+  constexpr int BM = 32 * MT;
+  __shared__ __align__(16) uint32_t lds[GemmLds<F, MT, KS>::DWORDS];
+  __shared__ int sxr[BM], syr[BM];
+  const int t = threadIdx.x;
   const uint8_t* wb = a.w;
   const float* bias = a.bias;
   int nrows;
   if (a.items) {
-    const int4 it = a.items[blockIdx.y];
-    if (it.z <= 0) return;
+    // an item of up to 64 slots: 64 / BM blocks
+    constexpr int PARTS = 64 / BM;
+    const int4 it = a.items[blockIdx.y / PARTS];
+    const int r0 = (int)(blockIdx.y % PARTS) * BM;
+    if (it.z <= r0) return;
     wb += (int64_t)it.x * a.stride;
     if (bias) bias += (int64_t)it.x * a.out;
-    nrows = min(GBM, it.z);
-    if (t < GBM) {
-      const int sl = a.perm[it.y + min(t, nrows - 1)];
+    nrows = min(BM, it.z - r0);
+    if (t < BM) {
+      const int sl = a.perm[it.y + r0 + min(t, nrows - 1)];
       sxr[t] = a.x_per_slot ? sl / a.x_per_slot : 0;
       syr[t] = sl;
     }
   } else {
-    const int r0 = blockIdx.y * GBM;
-    nrows = min(GBM, a.rows - r0);
-    if (t < GBM) sxr[t] = syr[t] = r0 + min(t, nrows - 1);
+    const int r0 = blockIdx.y * BM;
+    nrows = min(BM, a.rows - r0);
+    if (t < BM) sxr[t] = syr[t] = r0 + min(t, nrows - 1);
   }
   __syncthreads();
-  const Regions rg = regions(F, a.out, a.in);
-  const int col0 = blockIdx.x * GBN;
-  const int o_real = col0 + 32 * wn + (l & 31);
-  const int64_t o = min(o_real, a.out - 1);
-  const int rb = 32 * wm + 4 * h;  // tile row of result register i: rb + 8 (i / 4) + i % 4
-  constexpr int WS = GKC * raw_dwords<F>() + 1;
-  const uint32_t* myw = sw_ + (32 * wn + (l & 31)) * WS;     // this lane's weight column
-  const uint32_t* mya = sa_ + (32 * wm + (l & 31)) * GSA;    // this lane's activation row
-
-  double acc[16];
-  int isum[16], msum[16];
-#pragma unroll
-  for (int i = 0; i < 16; i++) {
-    acc[i] = 0.0;
-    isum[i] = msum[i] = 0;
-  }
-  // Q4_K: the super-block's minimum sum sum_j m_j bsum_j kept on the matrix
-  // cores: A times the group's m_j broadcast (m < 64), accumulated over the
-  // 8 groups of the super-block, exact int32
-  v16i cm = {};
-
-  // chunk c + 1 is in registers (its loads issued during chunk c - 1) while
-  // chunk c is computed from LDS; loads past the last group read the last
-  // group (values unused)
-  const int nch = (G + GKC - 1) / GKC;
-  ChunkRegs cr;
-  chunk_load<F>(a, wb, rg, col0, sxr, xstride, G, 0, cr);
-  chunk_store<F>(cr, sw_, sa_, sdx_, sbs_);
-  chunk_load<F>(a, wb, rg, col0, sxr, xstride, G, GKC, cr);
-  __syncthreads();
-  for (int c = 0; c < nch; c++) {
-    const int gc = c * GKC;
-#pragma unroll
-    for (int j = 0; j < GKC; j++) {
-      const int g = gc + j;
-      if (g < G) {
-        const Raw r = raw_get<F>(myw + j, GKC);
-        const uint2 x0 = *(const uint2*)(mya + j * 8 + 2 * h);
-        const uint2 x1 = *(const uint2*)(mya + j * 8 + 4 + 2 * h);
-        double (*sdx)[GBM] = (double (*)[GBM])sdx_;
-        int (*sbs)[GBM] = (int (*)[GBM])sbs_;
-        const int buf = 0;
-        (void)buf;
-          const v4i bv = b_operand<F>(r, h);
-          v16i s;
-          v16i s2 = {};
-          if constexpr (F == DT_Q4_K) {
-            int sc, mn;
-            scale_min_k4(g & 7, r.q1.y, r.q1.z, r.q1.w, sc, mn);
-            const int mb = (int)(((uint32_t)mn * 0x010101u) | ((uint32_t)mn << 24));
-            const v4i bm = {mb, mb, mb, mb};
-            const v4i av = {(int)x0.x, (int)x0.y, (int)x1.x, (int)x1.y};
-            const v16i z = {};
-            s = __builtin_amdgcn_mfma_i32_32x32x32_i8(av, bv, z, 0, 0, 0);
-            cm = __builtin_amdgcn_mfma_i32_32x32x32_i8(av, bm, (g & 7) == 0 ? z : cm, 0, 0, 0);
-#pragma unroll
-            for (int i = 0; i < 16; i++) isum[i] += __mul24(sc, s[i]);  // |sums| < 2^16, sc < 64
-            if ((g & 7) == 7) {  // (Q4_K rows hold whole super-blocks)
-              const double hd = half_to_float(r.q1.x & 0xffffu), hm = half_to_float(r.q1.x >> 16);
-#pragma unroll
-              for (int i = 0; i < 16; i++) {
-                const double dx = sdx[j][rb + 8 * (i >> 2) + (i & 3)];
-                acc[i] = acc[i] + ((hd * dx) * (double)isum[i] - (hm * dx) * (double)cm[i]);
-                isum[i] = 0;
-              }
-            }
-            continue;
-          }
-          if constexpr (F == DT_Q6_K) {
-            // the two 16-value sub-blocks of the group, each its own sum
-            const v16i z = {};
-            s = __builtin_amdgcn_mfma_i32_32x32x16_i8(
-                (long)(((uint64_t)x0.y << 32) | x0.x),
-                (long)(((uint64_t)(uint32_t)bv.y << 32) | (uint32_t)bv.x), z, 0, 0, 0);
-            s2 = __builtin_amdgcn_mfma_i32_32x32x16_i8(
-                (long)(((uint64_t)x1.y << 32) | x1.x),
-                (long)(((uint64_t)(uint32_t)bv.w << 32) | (uint32_t)bv.z), z, 0, 0, 0);
-          } else {
-            const v4i av = {(int)x0.x, (int)x0.y, (int)x1.x, (int)x1.y};
-            const v16i z = {};
-            s = __builtin_amdgcn_mfma_i32_32x32x32_i8(av, bv, z, 0, 0, 0);
-          }
-          // the group's terms (group_q8 / group_q8k / superblock_q8k)
-          if constexpr (F == DT_Q4_K) {
-            int sc, mn;
-            scale_min_k4(g & 7, r.q1.y, r.q1.z, r.q1.w, sc, mn);
-#pragma unroll
-            for (int i = 0; i < 16; i++) {
-              // |sums| < 2^16, scales < 64: 24-bit multiplies
-              isum[i] += __mul24(sc, s[i]);
-              msum[i] += __mul24(mn, sbs[j][rb + 8 * (i >> 2) + (i & 3)]);
-            }
-            if ((g & 7) == 7) {
-              const double hd = half_to_float(r.q1.x & 0xffffu), hm = half_to_float(r.q1.x >> 16);
-#pragma unroll
-              for (int i = 0; i < 16; i++) {
-                const double dx = sdx[j][rb + 8 * (i >> 2) + (i & 3)];
-                acc[i] = acc[i] + ((hd * dx) * (double)isum[i] - (hm * dx) * (double)msum[i]);
-                isum[i] = msum[i] = 0;
-              }
-            }
-          } else if constexpr (F == DT_Q6_K) {
-            const int sa = (int)(int8_t)(r.a & 255u), sb = (int)(int8_t)(r.a >> 8);
-#pragma unroll
-            for (int i = 0; i < 16; i++) isum[i] += __mul24(sa, s[i]) + __mul24(sb, s2[i]);
-            if ((g & 7) == 7) {
-              const double d = half_to_float(r.d);
-#pragma unroll
-              for (int i = 0; i < 16; i++) {
-                const double dx = sdx[j][rb + 8 * (i >> 2) + (i & 3)];
-                acc[i] = acc[i] + (d * dx) * (double)isum[i];
-                isum[i] = 0;
-              }
-            }
-          } else if constexpr (F == DT_Q5_1) {
-            const double d = half_to_float(r.a & 0xffffu), m = half_to_float(r.a >> 16);
-#pragma unroll
-            for (int i = 0; i < 16; i++) {
-              const int ri = rb + 8 * (i >> 2) + (i & 3);
-              const double dx = sdx[j][ri];
-              const double tt = (double)s[i] * (d * dx);
-              acc[i] = acc[i] + (tt + m * (dx * (double)sbs[j][ri]));
-            }
-          } else {
-            double dw;
-            if constexpr (F == DT_MXFP4) dw = mxfp4_q8_scale(r.a);
-            else dw = half_to_float(r.a);
-            // s * dw * dx is exact in double (at most 19 + 11 + 11 significant
-            // bits), so one fused multiply-add rounds as the CPU's multiply-then-add
-            // the 16 rows' scales: four 16-byte LDS reads, all issued first
-            double2 dq[8];
-#pragma unroll
-            for (int q = 0; q < 8; q++) dq[q] = *(const double2*)&sdx[j][rb + 8 * (q >> 1) + 2 * (q & 1)];
-#pragma unroll
-            for (int i = 0; i < 16; i++) {
-              const double2 d2 = dq[i >> 1];
-              const double dx = (i & 1) ? d2.y : d2.x;
-              acc[i] = __builtin_fma((double)s[i], dw * dx, acc[i]);
-            }
-          }
-      }
-    }
-    __syncthreads();  // the chunk's LDS reads are done
-    chunk_store<F>(cr, sw_, sa_, sdx_, sbs_);
-    chunk_load<F>(a, wb, rg, col0, sxr, xstride, G, gc + 2 * GKC, cr);
-    __syncthreads();
-  }
-  if (o_real >= a.out) return;
-  const double b = bias ? (double)bias[o] : 0.0;
-#pragma unroll
-  for (int i = 0; i < 16; i++) {
-    const int rt = rb + 8 * (i >> 2) + (i & 3);
-    if (rt < nrows) {
-      double v = acc[i];
-      if (bias) v = b + v;
-      a.y[(int64_t)syr[rt] * a.out + o] = (float)v;
+  // an item (or a last tile) of at most 32 rows needs one tile a wave
+  if constexpr (MT == 2) {
+    if (nrows <= 32) {
+      gemm_tiles<F, 1, KS>(a, wb, bias, nrows, sxr, syr, lds);
+      return;
     }
   }
+  gemm_tiles<F, MT, KS>(a, wb, bias, nrows, sxr, syr, lds);
 }
 
 // ------------------------------------------------ a small batch of rows
@@ -666,7 +873,7 @@ __device__ __forceinline__ void chunk8_store(const Chunk8& cr, uint32_t* sw, uin
   for (int p = 0; p < 4; p++) raw_put<F>(sw + ((t >> 3) + 32 * p) * WS + (t & 7), GKC, cr.wr[p]);
   if (t < 64) {
     const int row = t >> 3, j = t & 7;
-    uint32_t* d = sa + row * GSA + j * 8;
+    uint32_t* d = sa + row * G8A + j * 8;
     *(v4u32*)d = cr.xc[0];
     *(v4u32*)(d + 4) = cr.xc[1];
     sdx[j * 8 + row] = cr.dx;
@@ -687,7 +894,7 @@ __device__ __forceinline__ void gemm8(const GemmArgs& a)
 {
   constexpr int WS = GKC * raw_dwords<F>() + 1;
   __shared__ uint32_t sw_[G8N * WS];
-  __shared__ __align__(16) uint32_t sa_[8 * GSA];
+  __shared__ __align__(16) uint32_t sa_[8 * G8A];
   __shared__ __align__(16) float sdx_[GKC * 8];
   __shared__ int sbs_[needs_xsum(F) ? GKC * 8 : 1];
   __shared__ int sxr[8], syr[8];
@@ -724,7 +931,7 @@ __device__ __forceinline__ void gemm8(const GemmArgs& a)
   if (nsteps == 0) return;
   const int arow = l & 31;  // A lane: row arow (rows 8.. are zero)
   const uint32_t* myw = sw_ + (32 * w + (l & 31)) * WS;
-  const uint32_t* mya = sa_ + min(arow, 7) * GSA;
+  const uint32_t* mya = sa_ + min(arow, 7) * G8A;
   auto step_at = [&](int q, int& col0, int& gc) {
     col0 = ((int)blockIdx.x + (q / nch) * (int)gridDim.x) * G8N;
     gc = (q % nch) * GKC;
@@ -992,10 +1199,20 @@ __device__ __forceinline__ void gemm_flt(const GemmArgs& a)
 
 }  // namespace ihip
 
-// (three blocks a CU: the registers fit in 168, no spill; a b512 6144 x 2048
-// launch's 768 blocks then run in one round instead of one and a half)
-#define IHIP_GEMM(NAME, F)                                                                      \
-  extern "C" __global__ __launch_bounds__(256, 3) void gemm_##NAME(ihip::GemmArgs a) { ihip::gemm<F>(a); } \
+#define IHIP_GEMM_TILES(NAME, F, MT, KS)                                                            \
+  extern "C" __global__ __launch_bounds__(256, 2) void gemm_##NAME##_m##MT##k##KS(ihip::GemmArgs a) \
+  {                                                                                                 \
+    ihip::gemm<F, MT, KS>(a);                                                                       \
+  }
+// (64-row tiles share a K-quant's decode between two MFMA tiles; the formats
+// of 32 values would spill in them, two doubles an output and group)
+#define IHIP_GEMM_K(NAME, F)     \
+  IHIP_GEMM_TILES(NAME, F, 2, 1) \
+  IHIP_GEMM(NAME, F)
+#define IHIP_GEMM(NAME, F)                                                                          \
+  IHIP_GEMM_TILES(NAME, F, 1, 1)                                                                    \
+  IHIP_GEMM_TILES(NAME, F, 1, 2)                                                                    \
+  IHIP_GEMM_TILES(NAME, F, 1, 4)                                                                    \
   extern "C" __global__ __launch_bounds__(256) void gemm8_##NAME(ihip::GemmArgs a)                    \
   {                                                                                                 \
     ihip::touch_kernargs<sizeof(ihip::GemmArgs)>();                                                 \
@@ -1032,8 +1249,8 @@ IHIP_GEMM(q5_0, ihip::DT_Q5_0)
 IHIP_GEMM(q5_1, ihip::DT_Q5_1)
 #endif
 #ifdef IHIP_ONLY_FMT_Q4_K
-IHIP_GEMM(q4_k, ihip::DT_Q4_K)
+IHIP_GEMM_K(q4_k, ihip::DT_Q4_K)
 #endif
 #ifdef IHIP_ONLY_FMT_Q6_K
-IHIP_GEMM(q6_k, ihip::DT_Q6_K)
+IHIP_GEMM_K(q6_k, ihip::DT_Q6_K)
 #endif

@@ -1,0 +1,69 @@
+"""The prompt GEMM's block shapes (gemm.hip: 32 or 64 rows by 128, 64 or 32
+outputs, the sum whole or in 2 or 4 parts) and the rule that takes them, at
+their edges: one row and output past a tile, sums of one group, of a part of
+a chunk and of chunks that leave waves idle, rows around the 8-row launches'
+limit, against the CPU oracle's Linear.
+
+Bound: the group sums are exact integers and the scales multiply in double, so
+only the order of a double sum differs from the CPU's: a value differs by at
+most one ulp of single, in at most 1/1000 of the values (the bound of the
+other Linear tests)."""
+import numpy as np
+import pytest
+
+import infer_hip as H
+import oracle_lib as O
+
+pytestmark = pytest.mark.gpu
+
+BLOCK = [H.Q8_0, H.Q4_0, H.MXFP4, H.Q5_0, H.Q5_1, H.Q4_K, H.Q6_K]
+# (rows, in, out): four shapes of tiles, the edges of the rule between them
+SHAPES = [(9, 32, 6144), (9, 256, 3073), (12, 288, 3200), (17, 2048, 2100), (33, 1056, 1025),
+          (80, 512, 33), (81, 3328, 129), (97, 1280, 8193), (257, 768, 4100), (1024, 256, 2049),
+          (1023, 544, 4097)]
+
+
+@pytest.fixture(scope="module")
+def ctx():
+    c = H.Context(0)
+    yield c
+    c.close()
+
+
+@pytest.mark.parametrize("dtype", BLOCK, ids=[H.NAMES[t] for t in BLOCK])
+def test_tiles_match_oracle(ctx, dtype):
+    for rows, cols, out in SHAPES:
+        if cols % H.BLOCK[dtype][0]:
+            cols = -(-cols // 256) * 256
+        rng = np.random.default_rng(rows + out)
+        x = rng.standard_normal((rows, cols)).astype(np.float32)
+        x[:, ::61] *= 9
+        x[rows // 2] = 0
+        bias = rng.standard_normal(out).astype(np.float32)
+        w = H.synth_blocks(dtype, out, cols, rows + cols, -8, -4)
+        got = ctx.linear(x, w, dtype, out, bias, mode=H.MODE_Q8)
+        ref = O.linear(x, w, dtype, out, bias)
+        bits = np.abs(got.view(np.int32).astype(np.int64) - ref.view(np.int32).astype(np.int64))
+        print(H.NAMES[dtype], rows, cols, out, "differ", int((bits > 0).sum()), flush=True)
+        # (a value within a rounding of zero may change its sign bit: compared by size)
+        near = np.abs(got - ref) <= np.abs(ref) * 2.0 ** -23 + 1e-30
+        assert np.all((bits <= 1) | near), (rows, cols, out, int(bits.max()))
+        assert (bits > 0).mean() <= 1e-3
+
+
+def test_quantized_input_and_rows_apart(ctx):
+    # a row's result does not depend on the rows beside it, nor on who
+    # quantized it
+    rows, cols, out = 75, 1024, 2500
+    x = np.random.default_rng(3).standard_normal((rows, cols)).astype(np.float32)
+    w = H.synth_blocks(H.Q4_K, out, cols, 5, -8, -4)
+    dw = ctx.weight(w, H.Q4_K, out, cols)
+    L = H.lib()
+    dx, y, q = ctx.array(x), ctx.alloc(rows * out * 4), ctx.alloc(rows * int(L.ihip_q8_bytes(cols, 1)))
+    H.check(L.ihip_enqueue_quantize(ctx.h, dx.ptr, rows, cols, 1, q.ptr, 0))
+    H.check(L.ihip_enqueue_linear_at(ctx.h, q.ptr, rows, cols, H.Q4_K, dw, out, y.ptr, 0,
+                                     H.MODE_Q8 | 2))
+    ctx.sync()
+    a = y.download(np.float32, rows * out).reshape(rows, out)
+    assert np.array_equal(a, ctx.linear(x, w, H.Q4_K, out, mode=H.MODE_Q8))
+    assert np.array_equal(a[32:64], ctx.linear(x[32:64], w, H.Q4_K, out, mode=H.MODE_Q8))
