@@ -1259,11 +1259,18 @@ int enqueue_attention(ihip_ctx* c, uint64_t q, uint64_t kc, uint64_t vc, uint64_
          (const int*)pastp, (double*)part, scale, (int32_t)rows, (int32_t)heads, (int32_t)kvh,
          (int32_t)hd, (int32_t)past, (int32_t)window, f16, splits};
   int rc;
-  if ((hd == 64 || hd == 128) && rows > 1 && c->attn_mfma) {
-    // tiles of 16 rows on the f64 matrix cores
+  if ((hd == 64 || hd == 128 || hd == 256) && rows > 1 && c->attn_mfma && kvh * hd < 1 << 22) {
+    // tiles of 16 rows on the f64 matrix cores, a block per tile and head when
+    // these give every CU two, else the tile's key ranges in as many groups
+    // (with a merge) as do; the offsets inside a range are 24-bit products
+    // of its rows' bytes
+    const int64_t tiles = heads * ((rows + 15) / 16);
+    const int groups = (int)std::min<int64_t>(splits, tiles >= 2 * c->cus ? 1 : (2 * c->cus + tiles - 1) / tiles);
+    a.splits = groups;
     char name[32];
     snprintf(name, sizeof name, "attention_mfma_%s_%d", f16 ? "f16" : "f32", (int)hd);
-    rc = launch(c, name, dim3((unsigned)heads, (unsigned)((rows + 15) / 16), (unsigned)splits), dim3(256), &a);
+    rc = launch(c, name, dim3((unsigned)heads, (unsigned)((rows + 15) / 16), (unsigned)groups), dim3(256), &a);
+    if (rc || groups == 1) return rc;
   } else if ((hd == 64 || hd == 128) && rows > 1) {
     // tiles of 8 rows sharing each range's keys
     char name[32];

@@ -1054,88 +1054,128 @@ extern "C" __global__ __launch_bounds__(256) void attention_rows_f32_128(AttnArg
   attention_rows_t<false, 128>(a);
 }
 
-// The ranges of ATTM rows at once on the f64 matrix cores (prompt chunks,
-// head_dim HD = 64 or 128): one block per (head, tile of ATTM = 16
-// consecutive rows, range s), the rows' ranges as attention_rows forms them
-// (a tile's keys span at most ATT_CHUNK + 15). Scores Q K^T and the weighted
-// values P V are v_mfma_f64_16x16x4f64 products: q (float), the cached keys
-// and values (half or float) and the weights are exact as doubles, every
-// product is exact and the sums run in double - only their order differs
-// from the CPU's sequential dot (CausalRows, backend.cpu.pas:1305-1354), a
-// difference of the order of 1e-16 relative before the result is rounded
-// to single. Per MFMA, lane l holds A[l % 16][l / 16] and B[l / 16][l % 16];
-// D[l / 16 + 4 v][l % 16] comes back in its register v. The k index of a
-// lane group (l / 16) runs over a contiguous quarter of the dimensions (the
-// scores) or of the tile's keys (the values), so each lane reads its own
-// contiguous part of a row: the sum is over the same terms, permuted.
+// ATTM rows of a prompt chunk on the f64 matrix cores (head_dim HD = 64, 128
+// or 256): one block per (head, tile of ATTM = 16 consecutive rows, group s of
+// the tile's key ranges), walking its ranges of ATT_CHUNK keys with a running
+// maximum and sum per row, in double. With one group the block writes the
+// output itself; else its partial result, for attention_merge. Scores Q K^T
+// and the weighted values P V are v_mfma_f64_16x16x4f64 products: q (float),
+// the cached keys and values (half or float) and the weights are exact as
+// doubles, every product is exact and the sums run in double - only their
+// order differs from the CPU's sequential dot (CausalRows,
+// backend.cpu.pas:1305-1354), a difference of the order of 1e-16 relative
+// before the result is rounded to single. Per MFMA, lane l holds
+// A[l % 16][l / 16] and B[l / 16][l % 16]; D[l / 16 + 4 v][l % 16] comes back
+// in its register v. The k index of a lane group (l / 16) runs over a
+// contiguous quarter of the dimensions (the scores) or of the range's keys
+// (the values), so each lane reads its own contiguous part of a row: the sum
+// is over the same terms, permuted.
+//
+// Bound by the f64 matrix cores (4 hd operations a row and key, a 64-cycle
+// MFMA per 2048: 111 of the 188 us below) and the vector instructions beside
+// them, which the counters show in sequence with them rather than under them:
+// hence e^x of its own (exp_below), a row's softmax over 16 lanes, 24-bit
+// offsets for the values. A block per range before this wrote 130 doubles
+// a row, head and range, 272 MB for 1024 rows of 32 heads, and half of its
+// blocks lay past the causal end: 1024 rows from an empty cache, 32 heads of
+// 128, 331 us (ranges and merge) before, 188 now; 1000 rows, a window
+// of 128, 64 heads of 64: 147, 75 now; heads of 256 (512 rows, 8 heads) 162 on
+// attention_part and its merge, 64 now.
 constexpr int ATTM = 16;
-constexpr int ATTMK = ATT_CHUNK + ATTM;  // keys of a tile's range, padded to 16
+constexpr int ATTMK = ATT_CHUNK + ATTM;  // keys of a range at most, a multiple of 16
 typedef double dbl4 __attribute__((ext_vector_type(4)));
+
+// e^x for x <= 0 (or a NaN, which stays one): x = n ln 2 + r, |r| <= ln 2 / 2,
+// the Taylor sum of e^r to r^13 (its remainder below 2^-57) times 2^n. Within
+// an ulp of double, in half the instructions of the library's exp, which a
+// prompt's scores take as much time for as their products.
+__device__ __forceinline__ double exp_below(double x)
+{
+  x = x < -800.0 ? -800.0 : x;  // 0 from -745.2 on
+  const double n = __builtin_rint(x * 1.4426950408889634);
+  // ln 2 as a double and what it lacks
+  double r = __builtin_fma(n, -0.6931471805599453, x);
+  r = __builtin_fma(n, -2.3190468138462996e-17, r);
+  double p = 1.0 / 6227020800.0;  // 1 / 13!
+  p = __builtin_fma(p, r, 1.0 / 479001600.0);
+  p = __builtin_fma(p, r, 1.0 / 39916800.0);
+  p = __builtin_fma(p, r, 1.0 / 3628800.0);
+  p = __builtin_fma(p, r, 1.0 / 362880.0);
+  p = __builtin_fma(p, r, 1.0 / 40320.0);
+  p = __builtin_fma(p, r, 1.0 / 5040.0);
+  p = __builtin_fma(p, r, 1.0 / 720.0);
+  p = __builtin_fma(p, r, 1.0 / 120.0);
+  p = __builtin_fma(p, r, 1.0 / 24.0);
+  p = __builtin_fma(p, r, 1.0 / 6.0);
+  p = __builtin_fma(p, r, 0.5);
+  p = __builtin_fma(p, r, 1.0);
+  p = __builtin_fma(p, r, 1.0);
+  return __builtin_ldexp(p, (int)n);
+}
 
 template <bool F16, int HD>
 __device__ __forceinline__ void attention_mfma_t(const AttnArgs& a)
 {
-  __shared__ double sc[ATTM][ATTMK + 1];  // scores, then weights (row, tile key)
-  __shared__ double stat[ATTM][2];
-  __shared__ int rk[ATTM][2];             // a row's keys [k0, k1) (absolute)
-  const int h = xcd_head(blockIdx.x, a.heads), r0 = blockIdx.y * ATTM, s = blockIdx.z;
+  __shared__ double sc[2][ATTM][ATTMK + 1];  // scores, then weights (row, key of the range)
+  __shared__ double stat[ATTM][2];           // a row's running maximum and sum
+  __shared__ double shrink[ATTM];            // exp(old maximum - new maximum)
+  const int h = xcd_head(blockIdx.x, a.heads), s = blockIdx.z;
+  // the tiles with the most keys first
+  const int r0 = (int)(gridDim.y - 1 - blockIdx.y) * ATTM;
   const int t = threadIdx.x, w = t >> 6, l = t & 63, lq = l >> 4, lc = l & 15;
   constexpr int d = HD;
   const int64_t kvw = (int64_t)a.kvh * d, qw = (int64_t)a.heads * d;
   const int g = h / (a.heads / a.kvh);
   const int past = a.pastp ? *a.pastp : a.past;
-  if (t < ATTM) {
-    const int r = t;
+  // row r sees the keys [first(r), past + r0 + r]; the tile's keys [kb, kend)
+  // in nit ranges, this group's [it0, it1)
+  const int rlast = min(ATTM, a.rows - r0) - 1;
+  auto first = [&](int r) __attribute__((always_inline)) {
     const int total = past + r0 + r + 1;
-    const int first = (a.window > 0 && total > a.window) ? total - a.window : 0;
-    const int cnt = total - first;
-    const int j0 = min(cnt, s * ATT_CHUNK), j1 = min(cnt, j0 + ATT_CHUNK);
-    int k0 = first + j0, k1 = first + j1;
-    if (r0 + r >= a.rows || k0 >= k1) k0 = k1 = -1;  // no key of this range
-    rk[r][0] = k0;
-    rk[r][1] = k1;
+    return a.window > 0 && total > a.window ? total - a.window : 0;
+  };
+  const int kb0 = first(0), kend = past + r0 + rlast + 1, span = kend - kb0;
+  const int per = span <= ATTMK ? ATTMK : ATT_CHUNK;
+  const int nit = (span + per - 1) / per;
+  const int it0 = s * nit / a.splits, it1 = (s + 1) * nit / a.splits;
+  if (t < ATTM) {
+    stat[t][0] = -1.0e308;
+    stat[t][1] = 0.0;
   }
-  __syncthreads();
-  // the tile's keys [kb, ke): from the first row with keys to the last
-  int kb = 0x7fffffff, ke = -1;
+  constexpr int DQ = d / 4;  // scores: k steps = a lane's dimensions
+  float qa[DQ];  // (widened at each use: as doubles they halve the waves a SIMD holds)
+  {
+    const int qr = r0 + min(lc, rlast);
+    const float4* qp = (const float4*)(a.q + (int64_t)qr * qw + (int64_t)h * d + lq * DQ);
 #pragma unroll
-  for (int r = 0; r < ATTM; r++)
-    if (rk[r][0] >= 0) {
-      kb = min(kb, rk[r][0]);
-      ke = max(ke, rk[r][1]);
+    for (int i = 0; i < DQ / 4; i++) {
+      const float4 u = qp[i];
+      qa[4 * i] = u.x;
+      qa[4 * i + 1] = u.y;
+      qa[4 * i + 2] = u.z;
+      qa[4 * i + 3] = u.w;
     }
-  const int nblk = ke > kb ? (ke - kb + 15) >> 4 : 0;  // blocks of 16 keys (<= 9)
-  if (nblk > 0) {
+  }
+  constexpr int NT = d / 64;  // values: dimensions of a lane, one per tile
+  const int dim0 = w * (d / 4) + NT * lc;
+  dbl4 o[NT];
+#pragma unroll
+  for (int n = 0; n < NT; n++) o[n] = dbl4{0.0, 0.0, 0.0, 0.0};
+  __syncthreads();
+  for (int it = it0; it < it1; it++) {
+    const int kb = kb0 + it * per, ke = min(kend, kb + per);
+    const int nblk = (ke - kb + 15) >> 4, nk = 16 * nblk;  // blocks of 16 keys (<= 9)
+    double (*p)[ATTMK + 1] = sc[it & 1];
     // ---- scores: wave w takes key blocks w, w + 4, w + 8; lane group lq
     // the dimensions [lq * d / 4, (lq + 1) * d / 4)
-    constexpr int DQ = d / 4;  // k steps = a lane's dimensions
-    const int qr = min(r0 + lc, a.rows - 1);
-    double qa[DQ];
-    {
-      const float4* qp = (const float4*)(a.q + (int64_t)qr * qw + (int64_t)h * d + lq * DQ);
-#pragma unroll
-      for (int i = 0; i < DQ / 4; i++) {
-        const float4 u = qp[i];
-        qa[4 * i] = u.x;
-        qa[4 * i + 1] = u.y;
-        qa[4 * i + 2] = u.z;
-        qa[4 * i + 3] = u.w;
-      }
-    }
     for (int kbk = w; kbk < nblk; kbk += 4) {
       const int key = min(kb + 16 * kbk + lc, ke - 1);
       const int64_t kr = (int64_t)key * kvw + (int64_t)g * d + lq * DQ;
       constexpr int NW = F16 ? DQ / 8 : DQ / 4;  // 16-byte words of a lane's part
+      const uint4* kp = F16 ? (const uint4*)((const uint16_t*)a.kc + kr) : (const uint4*)((const float*)a.kc + kr);
       uint4 u[NW];
-      if constexpr (F16) {
-        const uint4* p = (const uint4*)((const uint16_t*)a.kc + kr);
 #pragma unroll
-        for (int i = 0; i < NW; i++) u[i] = p[i];
-      } else {
-        const uint4* p = (const uint4*)((const float*)a.kc + kr);
-#pragma unroll
-        for (int i = 0; i < NW; i++) u[i] = p[i];
-      }
+      for (int i = 0; i < NW; i++) u[i] = kp[i];
       dbl4 acc = {0.0, 0.0, 0.0, 0.0};
 #pragma unroll
       for (int i = 0; i < NW; i++) {
@@ -1143,127 +1183,177 @@ __device__ __forceinline__ void attention_mfma_t(const AttnArgs& a)
 #pragma unroll
         for (int j = 0; j < 4; j++) {
           if constexpr (F16) {
-            acc = __builtin_amdgcn_mfma_f64_16x16x4f64(qa[8 * i + 2 * j], (double)half_to_float(wv[j] & 0xffffu), acc, 0, 0, 0);
-            acc = __builtin_amdgcn_mfma_f64_16x16x4f64(qa[8 * i + 2 * j + 1], (double)half_to_float(wv[j] >> 16), acc, 0, 0, 0);
+            acc = __builtin_amdgcn_mfma_f64_16x16x4f64((double)qa[8 * i + 2 * j],
+                                                       (double)half_to_float(wv[j] & 0xffffu), acc, 0, 0, 0);
+            acc = __builtin_amdgcn_mfma_f64_16x16x4f64((double)qa[8 * i + 2 * j + 1],
+                                                       (double)half_to_float(wv[j] >> 16), acc, 0, 0, 0);
           } else {
-            acc = __builtin_amdgcn_mfma_f64_16x16x4f64(qa[4 * i + j], (double)bits_float(wv[j]), acc, 0, 0, 0);
+            acc = __builtin_amdgcn_mfma_f64_16x16x4f64((double)qa[4 * i + j], (double)bits_float(wv[j]), acc, 0, 0, 0);
           }
         }
       }
       // D[row][key]: row lq + 4 v, key column lc of this block
-      const int kk = 16 * kbk + lc, kabs = kb + kk;
+      const int kabs = kb + 16 * kbk + lc;
 #pragma unroll
       for (int v = 0; v < 4; v++) {
         const int r = lq + 4 * v;
-        const bool in = kabs >= rk[r][0] && kabs < rk[r][1];
-        sc[r][kk] = in ? acc[v] * a.scale : -1.0e308;
+        const bool in = kabs < ke && kabs >= first(r) && kabs <= past + r0 + r;
+        p[r][16 * kbk + lc] = in ? acc[v] * a.scale : -1.0e308;
       }
     }
-  }
-  __syncthreads();
-  const int nk = 16 * nblk;
-  // ---- per row: the range maximum, the weights exp(score - max), their sum
-  // (wave w takes rows 4w .. 4w + 3)
+    __syncthreads();
+    // ---- per row: the new maximum, the weights exp(score - max), the sum
+    // (row 4 w + lq over the 16 lanes of its lane group, all rows at once)
+    {
+      constexpr int NB = ATTMK / 16;
+      double* pr = p[4 * w + lq] + lc;
+      const double old = stat[4 * w + lq][0];
+      double x[NB], m = old;
 #pragma unroll
-  for (int rr = 0; rr < 4; rr++) {
-    const int r = 4 * w + rr;
-    double m = -1.0e308;
-    for (int j = l; j < nk; j += 64) m = fmax(m, sc[r][j]);
-    m = wave_max(m);
-    double e = 0;
-    for (int j = l; j < nk; j += 64) {
-      const double x = sc[r][j];
-      const double p = x > -1.0e308 ? exp(x - m) : 0.0;
-      sc[r][j] = p;
-      e += p;
-    }
-    e = wave_sum(e, 64);
-    if (l == 0) {
-      stat[r][0] = m;
-      stat[r][1] = e;
-    }
-  }
-  __syncthreads();
-  // ---- the weighted values: wave w the dimensions [w * d / 4, (w + 1) *
-  // d / 4) as NT tiles of 16 (HD 128: the even and the odd dimensions of the
-  // wave's 32); lane group lq the tile keys [lq * S, (lq + 1) * S)
-  constexpr int NT = d / 64;
-  const int S = nk >> 2;  // k steps (nk is a multiple of 16)
-  dbl4 o[NT];
+      for (int i = 0; i < NB; i++) {
+        x[i] = i < nblk ? pr[16 * i] : -1.0e308;
+        m = fmax(m, x[i]);
+      }
+      m = fmax(m, xpart<1>(m));
+      m = fmax(m, xpart<2>(m));
+      m = fmax(m, xpart<4>(m));
+      m = fmax(m, xpart<8>(m));
+      double e = 0;
 #pragma unroll
-  for (int n = 0; n < NT; n++) o[n] = dbl4{0.0, 0.0, 0.0, 0.0};
-  if (nblk > 0) {
-    const int dim0 = w * (d / 4) + NT * lc;  // this lane's column dimension(s)
-    const int64_t vb = (int64_t)g * d + dim0;
-    constexpr int VU = 12;  // value loads in flight per lane
+      for (int i = 0; i < NB; i++)
+        if (i < nblk) {
+          const double y = x[i] > -1.0e308 ? exp_below(x[i] - m) : 0.0;
+          pr[16 * i] = y;
+          e += y;
+        }
+      e = wave_sum(e, 16);
+      if (lc == 0) {
+        const double f = old > -1.0e308 ? exp_below(old - m) : 0.0;
+        shrink[4 * w + lq] = f;
+        stat[4 * w + lq][0] = m;
+        stat[4 * w + lq][1] = __builtin_fma(stat[4 * w + lq][1], f, e);
+      }
+    }
+    __syncthreads();
+    // ---- the weighted values: wave w the dimensions [w * d / 4, (w + 1) *
+    // d / 4) as NT tiles of 16 (the wave's dimensions modulo NT); lane group
+    // lq the range's keys [lq * S, (lq + 1) * S)
+    if (it > it0) {
+#pragma unroll
+      for (int v = 0; v < 4; v++) {
+        const double f = shrink[lq + 4 * v];
+#pragma unroll
+        for (int n = 0; n < NT; n++) o[n][v] *= f;
+      }
+    }
+    const int S = nk >> 2;  // k steps (nk is a multiple of 16)
+    constexpr int VU = NT > 2 ? 4 : 12;  // value loads in flight per lane
+    constexpr uint32_t ES = F16 ? 2 : 4;
+    // a uniform base and 24-bit products for the lane's offset (a range is at
+    // most ATTMK rows of kvw values)
+    const uint8_t* vbase = (const uint8_t*)a.vc + ((int64_t)kb * kvw + (int64_t)g * d) * ES;
+    const uint32_t vlast = (uint32_t)(ke - 1 - kb), vrow = (uint32_t)kvw * ES, vdim = (uint32_t)dim0 * ES;
     for (int t0 = 0; t0 < S; t0 += VU) {
       float vv[VU][NT];
 #pragma unroll
       for (int u = 0; u < VU; u++) {
-        const int key = min(kb + lq * S + min(t0 + u, S - 1), ke - 1);
-        const int64_t e = (int64_t)key * kvw + vb;
+        const uint8_t* vp = vbase + (__umul24(min((uint32_t)(lq * S + t0 + u), vlast), vrow) + vdim);
         if constexpr (F16) {
-          if constexpr (NT == 2) {
-            const uint32_t x = *(const uint32_t*)((const uint16_t*)a.vc + e);
-            vv[u][0] = half_to_float(x & 0xffffu);
-            vv[u][1] = half_to_float(x >> 16);
+          if constexpr (NT == 1) {
+            vv[u][0] = half_to_float(*(const uint16_t*)vp);
           } else {
-            vv[u][0] = half_to_float(((const uint16_t*)a.vc)[e]);
+            uint32_t x[NT / 2];
+            if constexpr (NT == 2) {
+              x[0] = *(const uint32_t*)vp;
+            } else {
+              const uint2 y = *(const uint2*)vp;
+              x[0] = y.x;
+              x[1] = y.y;
+            }
+#pragma unroll
+            for (int n = 0; n < NT; n++) vv[u][n] = half_to_float((n & 1) ? x[n / 2] >> 16 : x[n / 2] & 0xffffu);
           }
         } else {
-          if constexpr (NT == 2) {
-            const float2 x = *(const float2*)((const float*)a.vc + e);
+          if constexpr (NT == 1) {
+            vv[u][0] = *(const float*)vp;
+          } else if constexpr (NT == 2) {
+            const float2 x = *(const float2*)vp;
             vv[u][0] = x.x;
             vv[u][1] = x.y;
           } else {
-            vv[u][0] = ((const float*)a.vc)[e];
+            const float4 x = *(const float4*)vp;
+            vv[u][0] = x.x;
+            vv[u][1] = x.y;
+            vv[u][2] = x.z;
+            vv[u][3] = x.w;
           }
         }
       }
 #pragma unroll
       for (int u = 0; u < VU; u++) {
         if (t0 + u < S) {
-          const double p = sc[lc][lq * S + t0 + u];
+          const double x = p[lc][lq * S + t0 + u];
 #pragma unroll
           for (int n = 0; n < NT; n++)
-            o[n] = __builtin_amdgcn_mfma_f64_16x16x4f64(p, (double)vv[u][n], o[n], 0, 0, 0);
+            o[n] = __builtin_amdgcn_mfma_f64_16x16x4f64(x, (double)vv[u][n], o[n], 0, 0, 0);
         }
       }
     }
   }
-  // ---- the partial results: row lq + 4 v, dimension(s) dim0 + n
-  const int dim0 = w * (d / 4) + NT * lc;
+  // ---- row lq + 4 v, dimension(s) dim0 + n: the output, or the partial sums
+  // with the row's maximum and sum (an empty group: weight 0 in the merge)
 #pragma unroll
   for (int v = 0; v < 4; v++) {
     const int r = lq + 4 * v;
-    if (r0 + r >= a.rows) continue;
-    double* out = a.part + (((int64_t)h * a.rows + r0 + r) * a.splits + s) * (d + 2);
+    if (r > rlast) continue;
+    if (a.splits > 1) {
+      double* out = a.part + (((int64_t)h * a.rows + r0 + r) * a.splits + s) * (d + 2);
 #pragma unroll
-    for (int n = 0; n < NT; n++) out[dim0 + n] = o[n][v];
-  }
-  if (t < ATTM && r0 + t < a.rows) {
-    double* out = a.part + (((int64_t)h * a.rows + r0 + t) * a.splits + s) * (d + 2);
-    const bool empty = !(stat[t][1] > 0.0);
-    out[d] = empty ? -1.0e308 : stat[t][0];
-    out[d + 1] = empty ? 0.0 : stat[t][1];
+      for (int n = 0; n < NT; n++) out[dim0 + n] = o[n][v];
+      if (w == 0 && lc == 0) {
+        const bool empty = !(stat[r][1] > 0.0);
+        out[d] = empty ? -1.0e308 : stat[r][0];
+        out[d + 1] = empty ? 0.0 : stat[r][1];
+      }
+      continue;
+    }
+    double f = 1.0, den = stat[r][1];
+    if (a.sinks) {
+      const double sink = a.sinks[h], m = stat[r][0], top = fmax(m, sink);
+      f = exp(m - top);
+      den = __builtin_fma(den, f, exp(sink - top));
+    }
+    const double inv = 1.0 / den;
+    float* out = a.y + (int64_t)(r0 + r) * qw + (int64_t)h * d + dim0;
+#pragma unroll
+    for (int n = 0; n < NT; n++) out[n] = (float)(o[n][v] * f * inv);
   }
 }
 
-extern "C" __global__ __launch_bounds__(256) void attention_mfma_f16_64(AttnArgs a)
+extern "C" __global__ __launch_bounds__(256, 3) void attention_mfma_f16_64(AttnArgs a)
 {
   attention_mfma_t<true, 64>(a);
 }
-extern "C" __global__ __launch_bounds__(256) void attention_mfma_f16_128(AttnArgs a)
+extern "C" __global__ __launch_bounds__(256, 3) void attention_mfma_f16_128(AttnArgs a)
 {
   attention_mfma_t<true, 128>(a);
 }
-extern "C" __global__ __launch_bounds__(256) void attention_mfma_f32_64(AttnArgs a)
+extern "C" __global__ __launch_bounds__(256, 4) void attention_mfma_f32_64(AttnArgs a)
 {
   attention_mfma_t<false, 64>(a);
 }
-extern "C" __global__ __launch_bounds__(256) void attention_mfma_f32_128(AttnArgs a)
+extern "C" __global__ __launch_bounds__(256, 3) void attention_mfma_f32_128(AttnArgs a)
 {
   attention_mfma_t<false, 128>(a);
+}
+
+extern "C" __global__ __launch_bounds__(256, 2) void attention_mfma_f16_256(AttnArgs a)
+{
+  attention_mfma_t<true, 256>(a);
+}
+extern "C" __global__ __launch_bounds__(256, 2) void attention_mfma_f32_256(AttnArgs a)
+{
+  attention_mfma_t<false, 256>(a);
 }
 
 extern "C" __global__ __launch_bounds__(256) void attention_part_f16(AttnArgs a)

@@ -1,0 +1,55 @@
+"""The prompt attention over tiles of 16 rows (ops.hip attention_mfma_*): row
+counts and contexts at the edges of its tiles (16 rows) and ranges (128 keys,
+144 in one piece), windows that end inside a range, sinks, few tiles (the
+ranges in groups and a merge) and many (no merge), heads of 64, 128 and 256,
+half and float keys, against the CPU oracle.
+
+Bound: products and sums in double on both sides, e^x within an ulp of double;
+only their order differs, about 1e-15 relative for sums of 2000 weights before
+the one rounding to single: 2e-7 of the largest output allows two ulps."""
+import numpy as np
+import pytest
+
+import infer_hip as H
+import oracle_lib as O
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module")
+def ctx():
+    c = H.Context(0)
+    yield c
+    c.close()
+
+
+CASES = [  # heads, kv heads, head size, rows, past, window, sinks, half
+    (8, 2, 128, 2, 0, 0, False, True), (8, 2, 128, 16, 128, 0, False, True),
+    (4, 1, 128, 17, 127, 0, True, True), (8, 8, 128, 33, 1000, 0, False, False),
+    (8, 2, 64, 15, 129, 128, True, True), (16, 4, 64, 200, 300, 128, True, True),
+    (8, 2, 64, 144, 0, 16, False, False), (2, 1, 256, 31, 0, 0, False, True),
+    (4, 2, 256, 130, 513, 0, False, True), (4, 4, 256, 40, 700, 100, True, False),
+    (32, 4, 128, 600, 0, 0, False, True), (64, 8, 64, 150, 50, 0, False, False),
+    (8, 2, 256, 520, 0, 1024, False, True), (1, 1, 64, 3, 4000, 0, True, True)]
+
+
+@pytest.mark.parametrize("heads,kvh,hd,rows,past,window,sinks,half", CASES)
+def test_tiles_match_oracle(ctx, heads, kvh, hd, rows, past, window, sinks, half):
+    rng = np.random.default_rng(heads * rows + past)
+    total = past + rows
+    q = (rng.standard_normal((rows, heads * hd)) * 2).astype(np.float32)
+    k = rng.standard_normal((total, kvh * hd)).astype(np.float32)
+    v = rng.standard_normal((total, kvh * hd)).astype(np.float32)
+    k[total // 2] *= 8  # a key far above the others, in the middle of the ranges
+    if half:
+        k, v = k.astype(np.float16), v.astype(np.float16)
+    sk = rng.standard_normal(heads).astype(np.float32) if sinks else None
+    dq, dk, dv, y = ctx.array(q), ctx.array(k), ctx.array(v), ctx.alloc(q.nbytes)
+    ds = ctx.array(sk) if sinks else None
+    H.check(H.lib().ihip_enqueue_attention(ctx.h, dq.ptr, dk.ptr, dv.ptr, y.ptr, rows, heads, kvh,
+                                           hd, past, window, ds.ptr if ds else 0, 0.0, int(half)))
+    ctx.sync()
+    got = y.download(np.float32, rows * heads * hd).reshape(rows, heads * hd)
+    ref = O.causal_attention(q, heads, hd, k.astype(np.float32), v.astype(np.float32), past, kvh,
+                             window, sk)
+    assert np.abs(got - ref).max() <= 2e-7 * np.abs(ref).max()
