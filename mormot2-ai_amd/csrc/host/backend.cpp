@@ -457,7 +457,14 @@ int enqueue_linear(ihip_ctx* c, const LinearCall& k)
   // launches / GEMM: 16 rows of 2048 -> 6144 13.8 / 8.4, 16 of 1024 -> 3072
   // 7.5 / 6.9, 48 of 3072 -> 1024 10.9 / 10.9, 32 of it 9.5 / 11.0, 64 of
   // 2048 -> 512 8.2 / 9.2, 16 of 1024 -> 40000 20.4 / 11.3)
-  const bool few = q8 && c->gemm_few_rows && k.rows > 8 && (k.rows + 7) / 8 * k.out >= 6144;
+  // float weights: the 8-row launches' time grows with rows x weights, the
+  // GEMM's first 32 rows cost one tile (BF16, us, launches / GEMM: 4 rows of
+  // 2048 -> 6144 38.9 / 30.1, 2 rows 21 / 30; 8 rows of 3072 -> 1024 29.9 /
+  // 24.8, of 1024 -> 3072 22.2 / 19.5, of 2048 -> 512 13.0 / 18.5; 4 rows of
+  // 1024 -> 40000 94.8 / 90.9)
+  const int64_t elems = k.in * k.out;
+  const bool few = q8 ? c->gemm_few_rows && k.rows > 8 && (k.rows + 7) / 8 * k.out >= 6144
+                      : c->gemm_few_float && (k.rows >= 4 && elems >= 12 << 20 || k.rows >= 8 && elems >= 3 << 20);
   if (batch && gemm_q8 && (k.items ? k.item_rows > 8 : k.rows >= min_rows || few)) {
     struct {
       const uint8_t* w;
@@ -477,9 +484,11 @@ int enqueue_linear(ihip_ctx* c, const LinearCall& k)
            (const int*)k.perm, k.x_per_slot, 0, (const float*)k.x, nullptr, 1, 0};
     if (k.items && k.item_rows > 64) return fail(IHIP_E_ARG, "EnqueueLinear: items of at most 64 slots");
     char gname[32];
-    snprintf(gname, sizeof gname, "gemm_%s", fmt_name(k.dtype));
-    const unsigned gx = (unsigned)((k.out + 63) / 64);
-    const unsigned gy = (unsigned)(k.items ? k.nitems : (k.rows + 63) / 64);
+    const bool flt32 = float_fmt(k.dtype) && !k.items && k.rows <= 32;
+    const int64_t bm = flt32 ? 32 : 64;
+    snprintf(gname, sizeof gname, "gemm_%s_r%d", fmt_name(k.dtype), (int)bm);
+    const unsigned gx = (unsigned)((k.out + 4096 / bm - 1) / (4096 / bm));
+    const unsigned gy = (unsigned)(k.items ? k.nitems : (k.rows + bm - 1) / bm);
     // float weights with too few tiles to fill the chip (a router: 128
     // outputs): the sum split into ksplit parts of >= 256 values, one block
     // each, then their double sums added in split order

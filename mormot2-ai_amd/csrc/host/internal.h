@@ -76,6 +76,7 @@ struct ihip_ctx {
   int gemm_min_rows = ihip::GEMM_MIN_ROWS;  // the smallest chunk on the GEMM (IHIP_GEMM_MIN_ROWS)
   // 9 rows and more on the GEMM where its tiles pay (off with a chosen IHIP_GEMM_MIN_ROWS)
   bool gemm_few_rows = true;
+  bool gemm_few_float = true;  // the same for float weights (IHIP_GEMM_MIN_ROWS_FLOAT)
   // the smallest chunk of F32/BF16/F16 weights on the f64 GEMM
   // (IHIP_GEMM_MIN_ROWS_FLOAT)
   int gemm_min_rows_float = ihip::GEMM_MIN_ROWS_FLOAT;

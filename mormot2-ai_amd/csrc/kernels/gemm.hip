@@ -1072,29 +1072,61 @@ __device__ __forceinline__ void gemm8(const GemmArgs& a)
 // (backend.cpu.pas:1548-1565): every product of a float activation and a
 // float weight is exact in double, and the sum runs in double, here on the
 // f64 matrix cores (v_mfma_f64_16x16x4_f64; only the order of the double sum
-// differs from the CPU's). A block owns 64 rows x 64 outputs, each wave
-// 32 x 32 as 2 x 2 tiles of 16 x 16; chunks of FKC values of x and w are
-// loaded coalesced into LDS (the next chunk's loads in flight while one is
-// computed).
+// differs from the CPU's). A block owns BM rows x 4096 / BM outputs, each of
+// its 4 waves 32 x 32 as 2 x 2 tiles of 16 x 16; chunks of FKC values of x and
+// w are loaded as 16-byte words into LDS (the next chunk's loads in flight
+// while one is computed; in is a multiple of 32, so chunks are whole).
+//
+// A lane group's k values are a contiguous quarter of the chunk, so a lane
+// reads its 8 steps of a tile row as two 16-byte LDS words. Bound by the f64
+// matrix cores (a 64-cycle MFMA per 1024 products: 307 of the 717 us of 1024
+// rows 2880 -> 4096 before, when the operands came by 4-byte loads and LDS
+// reads; 442 now). 32 rows x 128 outputs for up to 32 rows, whose
+// matrix work is half a 64-row tile's.
 typedef double v4d __attribute__((ext_vector_type(4)));
-constexpr int FKC = 32;  // values of the sum per chunk
+constexpr int FKC = 32;       // values of the sum per chunk
+constexpr int FST = FKC + 4;  // LDS floats of a row's chunk
 
-template <int F>
-__device__ __forceinline__ float wval(const void* w, int64_t i)
+// N values from element i of float weights, widened
+template <int F, int N>
+__device__ __forceinline__ void wvals(const uint8_t* w, int64_t i, float (&v)[N])
 {
-  if constexpr (F == DT_F32) return ((const float*)w)[i];
-  else if constexpr (F == DT_BF16) return bits_float((uint32_t)((const uint16_t*)w)[i] << 16);
-  else return half_to_float(((const uint16_t*)w)[i]);
+  if constexpr (F == DT_F32) {
+    const v4u32* p = (const v4u32*)(w + i * 4);
+#pragma unroll
+    for (int k = 0; k < N / 4; k++) {
+      const v4u32 u = p[k];
+      v[4 * k] = bits_float(u.x);
+      v[4 * k + 1] = bits_float(u.y);
+      v[4 * k + 2] = bits_float(u.z);
+      v[4 * k + 3] = bits_float(u.w);
+    }
+  } else {
+    const v4u32* p = (const v4u32*)(w + i * 2);
+#pragma unroll
+    for (int k = 0; k < N / 8; k++) {
+      const v4u32 u = p[k];
+      const uint32_t q[4] = {u.x, u.y, u.z, u.w};
+#pragma unroll
+      for (int j = 0; j < 4; j++) {
+        v[8 * k + 2 * j] = F == DT_BF16 ? bits_float(q[j] << 16) : half_to_float(q[j] & 0xffffu);
+        v[8 * k + 2 * j + 1] = F == DT_BF16 ? bits_float(q[j] & 0xffff0000u) : half_to_float(q[j] >> 16);
+      }
+    }
+  }
 }
 
-template <int F>
+template <int F, int BM>
 __device__ __forceinline__ void gemm_flt(const GemmArgs& a)
 {
-  __shared__ float xs[2][GBM][FKC + 1];
-  __shared__ float ws[2][GBN][FKC + 1];
-  __shared__ int sxr[GBM], syr[GBM];
+  constexpr int BN = 4096 / BM;
+  constexpr int XT = 256 / BM, XN = FKC / XT;  // threads and values of a row's chunk
+  constexpr int WT = 256 / BN, WN = FKC / WT;
+  __shared__ __align__(16) float xs[2][BM][FST];
+  __shared__ __align__(16) float ws[2][BN][FST];
+  __shared__ int sxr[BM], syr[BM];
   const int t = threadIdx.x, l = t & 63, w = t >> 6;
-  const int wm = w & 1, wn = w >> 1;
+  const int wm = w % (BM / 32), wn = w / (BM / 32);
   const uint8_t* wb = a.w;
   const float* bias = a.bias;
   int nrows;
@@ -1103,74 +1135,88 @@ __device__ __forceinline__ void gemm_flt(const GemmArgs& a)
     if (it.z <= 0) return;
     wb += (int64_t)it.x * a.stride;
     if (bias) bias += (int64_t)it.x * a.out;
-    nrows = min(GBM, it.z);
-    if (t < GBM) {
+    nrows = min(BM, it.z);
+    if (t < BM) {
       const int sl = a.perm[it.y + min(t, nrows - 1)];
       sxr[t] = a.x_per_slot ? sl / a.x_per_slot : 0;
       syr[t] = sl;
     }
   } else {
-    const int r0 = blockIdx.y * GBM;
-    nrows = min(GBM, a.rows - r0);
-    if (t < GBM) sxr[t] = syr[t] = r0 + min(t, nrows - 1);
+    const int r0 = blockIdx.y * BM;
+    nrows = min(BM, a.rows - r0);
+    if (t < BM) sxr[t] = syr[t] = r0 + min(t, nrows - 1);
   }
   __syncthreads();
-  const int col0 = blockIdx.x * GBN;
-  // a thread's share of a chunk: 8 consecutive values of row (t / 4) of x
-  // and of column (t / 4) of w
-  const int lr = t >> 2, lk = 8 * (t & 3);
-  const float* xrow = a.x + (int64_t)sxr[lr] * a.in;
-  const int64_t wrow = (int64_t)min(col0 + lr, a.out - 1) * a.in;
+  const int col0 = blockIdx.x * BN;
   // this block's values of the sum: [kb, ke)
   const int kb = a.ksplit > 1 ? (int)blockIdx.z * a.klen : 0;
   const int ke = a.ksplit > 1 ? min(a.in, kb + a.klen) : a.in;
-  float xv[8], wv[8];
+  const int nch = (ke - kb) / FKC;  // (a split past the end: none)
+  // a thread's share of a chunk
+  const int xr = t / XT, xk = XN * (t % XT), wr = t / WT, wk = WN * (t % WT);
+  const float* xrow = a.x + (int64_t)sxr[xr] * a.in + xk;
+  const int64_t wrow = (int64_t)min(col0 + wr, a.out - 1) * a.in + wk;
+  float xv[XN], wv[WN];
   auto load = [&](int k0) __attribute__((always_inline)) {
 #pragma unroll
-    for (int u = 0; u < 8; u++) {
-      const int k = min(k0 + lk + u, ke - 1);
-      xv[u] = xrow[k];
-      wv[u] = wval<F>(wb, wrow + k);
+    for (int u = 0; u < XN / 4; u++) {
+      const float4 v = *(const float4*)(xrow + k0 + 4 * u);
+      xv[4 * u] = v.x;
+      xv[4 * u + 1] = v.y;
+      xv[4 * u + 2] = v.z;
+      xv[4 * u + 3] = v.w;
     }
+    wvals<F, WN>(wb, wrow + k0, wv);
   };
   auto store = [&](int buf) __attribute__((always_inline)) {
 #pragma unroll
-    for (int u = 0; u < 8; u++) {
-      xs[buf][lr][lk + u] = xv[u];
-      ws[buf][lr][lk + u] = wv[u];
-    }
+    for (int u = 0; u < XN; u += 4) *(float4*)&xs[buf][xr][xk + u] = make_float4(xv[u], xv[u + 1], xv[u + 2], xv[u + 3]);
+#pragma unroll
+    for (int u = 0; u < WN; u += 4) *(float4*)&ws[buf][wr][wk + u] = make_float4(wv[u], wv[u + 1], wv[u + 2], wv[u + 3]);
   };
   v4d acc[2][2];
 #pragma unroll
   for (int i = 0; i < 2; i++)
 #pragma unroll
     for (int j = 0; j < 2; j++) acc[i][j] = v4d{0.0, 0.0, 0.0, 0.0};
-  const int nch = (ke - kb + FKC - 1) / FKC;
-  load(kb);
-  store(0);
+  if (nch > 0) {
+    load(kb);
+    store(0);
+  }
   __syncthreads();
   // operand lane mapping of v_mfma_f64_16x16x4_f64 (probed on gfx950): A
   // lane l = row l % 16, k = l / 16; B lane l = column l % 16, k = l / 16;
   // result register e of lane l = row 4 e + l / 16, column l % 16
   const int ar = l & 15, ak = l >> 4;
   for (int c = 0; c < nch; c++) {
-    const int buf = c & 1, k0 = kb + c * FKC;
-    if (c + 1 < nch) load(k0 + FKC);
+    const int buf = c & 1;
+    if (c + 1 < nch) load(kb + (c + 1) * FKC);
+    const float* xp = &xs[buf][32 * wm + ar][8 * ak];
+    const float* wp = &ws[buf][32 * wn + ar][8 * ak];
 #pragma unroll
-    for (int kk = 0; kk < FKC; kk += 4) {
-      // a chunk past the end of the sum: values beyond in read 0 weight
-      const bool kin = k0 + kk + ak < ke;
-      double av[2], bv[2];
+    for (int q = 0; q < 8; q += 4) {
+      float4 av[2], bv[2];
 #pragma unroll
-      for (int i = 0; i < 2; i++) av[i] = (double)xs[buf][32 * wm + 16 * i + ar][kk + ak];
+      for (int i = 0; i < 2; i++) {
+        av[i] = *(const float4*)(xp + 16 * i * FST + q);
+        bv[i] = *(const float4*)(wp + 16 * i * FST + q);
+      }
 #pragma unroll
-      for (int j = 0; j < 2; j++) bv[j] = kin ? (double)ws[buf][32 * wn + 16 * j + ar][kk + ak] : 0.0;
+      for (int u = 0; u < 4; u++) {
+        double ad[2], bd[2];
 #pragma unroll
-      for (int i = 0; i < 2; i++)
+        for (int i = 0; i < 2; i++) {
+          ad[i] = u == 0 ? av[i].x : u == 1 ? av[i].y : u == 2 ? av[i].z : av[i].w;
+          bd[i] = u == 0 ? bv[i].x : u == 1 ? bv[i].y : u == 2 ? bv[i].z : bv[i].w;
+        }
 #pragma unroll
-        for (int j = 0; j < 2; j++) acc[i][j] = __builtin_amdgcn_mfma_f64_16x16x4f64(av[i], bv[j], acc[i][j], 0, 0, 0);
+        for (int i = 0; i < 2; i++)
+#pragma unroll
+          for (int j = 0; j < 2; j++) acc[i][j] = __builtin_amdgcn_mfma_f64_16x16x4f64(ad[i], bd[j], acc[i][j], 0, 0, 0);
+      }
     }
-    __syncthreads();
+    // (the other buffer was last read before the barrier that ended the chunk
+    // before)
     if (c + 1 < nch) store(buf ^ 1);
     __syncthreads();
   }
@@ -1219,8 +1265,15 @@ __device__ __forceinline__ void gemm_flt(const GemmArgs& a)
     ihip::gemm8<F>(a);                                                                              \
   }
 
-#define IHIP_GEMM_FLT(NAME, F) \
-  extern "C" __global__ __launch_bounds__(256) void gemm_##NAME(ihip::GemmArgs a) { ihip::gemm_flt<F>(a); }
+#define IHIP_GEMM_FLT(NAME, F)                                                               \
+  extern "C" __global__ __launch_bounds__(256, 4) void gemm_##NAME##_r64(ihip::GemmArgs a) \
+  {                                                                                          \
+    ihip::gemm_flt<F, 64>(a);                                                                \
+  }                                                                                          \
+  extern "C" __global__ __launch_bounds__(256, 4) void gemm_##NAME##_r32(ihip::GemmArgs a) \
+  {                                                                                          \
+    ihip::gemm_flt<F, 32>(a);                                                                \
+  }
 
 #ifdef IHIP_ONLY_FMT_Q8_0
 IHIP_GEMM(q8_0, ihip::DT_Q8_0)

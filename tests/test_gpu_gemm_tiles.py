@@ -67,3 +67,25 @@ def test_quantized_input_and_rows_apart(ctx):
     a = y.download(np.float32, rows * out).reshape(rows, out)
     assert np.array_equal(a, ctx.linear(x, w, H.Q4_K, out, mode=H.MODE_Q8))
     assert np.array_equal(a[32:64], ctx.linear(x[32:64], w, H.Q4_K, out, mode=H.MODE_Q8))
+
+
+# float weights (gemm_flt: tiles of 32 and 64 rows, the sum split over blocks
+# where there are few tiles): (rows, in, out) at the edges of tiles, chunks
+# of 32 values and splits
+FLOAT_SHAPES = [(4, 4096, 3100), (8, 3104, 1025), (17, 32, 33), (32, 1024, 129), (33, 1056, 65),
+                (64, 2080, 40), (65, 96, 4097), (200, 2880, 31)]
+
+
+@pytest.mark.parametrize("dtype", [H.F32, H.BF16, H.F16], ids=["F32", "BF16", "F16"])
+def test_float_tiles_match_oracle(ctx, dtype):
+    for rows, cols, out in FLOAT_SHAPES:
+        rng = np.random.default_rng(rows + out)
+        x = rng.standard_normal((rows, cols)).astype(np.float32)
+        bias = rng.standard_normal(out).astype(np.float32)
+        w = H.synth_normal(dtype, out, cols, rows + cols, 0.5)
+        got = ctx.linear(x, w, dtype, out, bias, mode=H.MODE_Q8)
+        ref = O.linear(x, w, dtype, out, bias)
+        bits = np.abs(got.view(np.int32).astype(np.int64) - ref.view(np.int32).astype(np.int64))
+        near = np.abs(got - ref) <= np.abs(ref) * 2.0 ** -23 + 1e-30
+        assert np.all((bits <= 1) | near), (rows, cols, out, int(bits.max()))
+        assert (bits > 0).mean() <= 1e-3
