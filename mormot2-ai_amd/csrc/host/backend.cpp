@@ -997,7 +997,7 @@ int ihip_enqueue_qkrope(ihip_ctx* c, uint64_t q, uint64_t k, uint64_t v, uint64_
   } a = {(float*)q, (const float*)k, (const float*)v, (const float*)qn, (const float*)kn,
          (const float*)cs, (void*)kc, (void*)vc, nullptr, eps, (int32_t)rows, (int32_t)heads,
          (int32_t)kvh, (int32_t)hd, (int32_t)past, kv_f16};
-  return launch(c, "qkrope", dim3((unsigned)(heads + kvh), (unsigned)rows), dim3(64), &a);
+  return launch_qkrope(c, hd, heads + kvh, rows, &a);
 }
 
 int ihip_enqueue_attention(ihip_ctx* c, uint64_t q, uint64_t kc, uint64_t vc, uint64_t y,
@@ -1187,6 +1187,13 @@ int attention_splits(int64_t maxkeys) { return (int)std::max<int64_t>(1, (maxkey
 
 // the ranges attention_merge weighs in one block
 static const int MAX_SPLITS = 256;
+
+int launch_qkrope(ihip_ctx* c, int64_t hd, int64_t heads, int64_t rows, void* args)
+{
+  const int per = rows > 1 ? 4 : 1;  // rows of a block, a wave each
+  return launch(c, hd <= 128 ? "qkrope_128" : hd <= 256 ? "qkrope_256" : "qkrope_512",
+                dim3((unsigned)heads, (unsigned)((rows + per - 1) / per)), dim3(64 * per), args);
+}
 
 int enqueue_attention_one(ihip_ctx* c, const AttnOne& o)
 {

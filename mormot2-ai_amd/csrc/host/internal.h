@@ -222,6 +222,8 @@ int enqueue_quantize(ihip_ctx* c, uint64_t x, int64_t rows, int64_t in, int kind
 // part holds heads * rows * splits * (hd + 2) doubles; pastp: the position
 // of row 0 in device memory (graph replay), or 0: past
 int attention_splits(int64_t maxkeys);
+// qkrope (its arguments at args) over `heads` q and kv heads of hd values
+int launch_qkrope(ihip_ctx* c, int64_t hd, int64_t heads, int64_t rows, void* args);
 // x += the k expert rows cd weighted by cw in slot order, then y = rmsnorm(x)
 int enqueue_addnorm_moe(ihip_ctx* c, uint64_t x, uint64_t cd, uint64_t cw, int64_t k, uint64_t w,
                         uint64_t y, int64_t rows, int64_t cols, double eps);

@@ -387,7 +387,7 @@ static int rope_attn(ihip_mctx* s, int l, int64_t n, int64_t past, bool graph)
           // the second set: every pair of the head (those beyond its share
           // have frequency 0)
           (int32_t)(L.rope_set ? 0 : rope_dims(d)), d.value_norm};
-  int rc = launch(m->c, "qkrope", dim3((unsigned)(d.heads + kvh), (unsigned)n), dim3(64), &ra);
+  int rc = launch_qkrope(m->c, hd, d.heads + kvh, n, &ra);
   if (rc) return rc;
   int64_t maxkeys = graph ? s->capacity : past + n;
   if (L.window > 0 && maxkeys > L.window) maxkeys = L.window;
@@ -1135,7 +1135,7 @@ static int layers(ihip_mctx* s, int64_t n, int64_t past, bool graph)
           int32_t slots, experts, max_items, chunk;
         } pa = {(const int*)s->ids_dev, (int*)s->perm, (void*)s->items, (int32_t)(n * K), (int32_t)E,
                 (int32_t)((n * K + m->item_rows - 1) / m->item_rows + E), m->item_rows};
-        if ((rc = launch(m->c, "moe_plan", dim3(1), dim3(256), &pa))) return rc;
+        if ((rc = launch(m->c, "moe_plan", dim3(1), dim3(1024), &pa))) return rc;
         // gate and up: slot s = row s / K, expert ids[s], grouped by expert
         bool q0 = false;
         if (m->mode == IHIP_MODE_Q8 && q8_kind(L.egd) >= 0) {

@@ -155,7 +155,7 @@ struct NormArgs {
 // registers and issues all their loads (and those of the k expert rows)
 // before the first sum, so a row costs one memory round trip.
 #define NORM_NV 4
-extern "C" __global__ __launch_bounds__(1024) void rmsnorm(NormArgs a)
+extern "C" __global__ __launch_bounds__(1024, 8) void rmsnorm(NormArgs a)
 {
   __shared__ double sh[16];
   const int64_t base = (int64_t)blockIdx.x * a.cols;
@@ -175,26 +175,31 @@ extern "C" __global__ __launch_bounds__(1024) void rmsnorm(NormArgs a)
       add[i] = 0.f;
     }
     if (a.cd) {
-      float cwv[16];
-      float cdv[16][NORM_NV];
+      // 8 slots at a time: with 16 in registers a CU held one block (the five
+      // norms of two MoE layers, 1024 rows of 2048 and 8 slots: 107 us in
+      // all, 68 now)
+      for (int j0 = 0; j0 < a.k; j0 += 8) {
+        float cwv[8];
+        float cdv[8][NORM_NV];
 #pragma unroll
-      for (int j = 0; j < 16; j++) {
-        int64_t sl = (int64_t)blockIdx.x * a.k + j;
-        cwv[j] = j < a.k ? a.cw[sl] : 0.f;
-#pragma unroll
-        for (int i = 0; i < NORM_NV; i++) {
-          int c = c0 + t + 1024 * i;
-          cdv[j][i] = (j < a.k && c < a.cols) ? a.cd[sl * a.cols + c] : 0.f;
-        }
-      }
-#pragma unroll
-      for (int j = 0; j < 16; j++)
-        if (j < a.k)
+        for (int j = 0; j < 8; j++) {
+          const int64_t sl = (int64_t)blockIdx.x * a.k + min(j0 + j, a.k - 1);
+          cwv[j] = a.cw[sl];
 #pragma unroll
           for (int i = 0; i < NORM_NV; i++) {
-            float p = cwv[j] * cdv[j][i];
-            add[i] = add[i] + p;
+            int c = c0 + t + 1024 * i;
+            cdv[j][i] = c < a.cols ? a.cd[sl * a.cols + c] : 0.f;
           }
+        }
+#pragma unroll
+        for (int j = 0; j < 8; j++)
+          if (j0 + j < a.k)
+#pragma unroll
+            for (int i = 0; i < NORM_NV; i++) {
+              float p = cwv[j] * cdv[j][i];
+              add[i] = add[i] + p;
+            }
+      }
     } else if (a.t) {
 #pragma unroll
       for (int i = 0; i < NORM_NV; i++) {
@@ -490,13 +495,18 @@ struct RopeArgs {
 // values (backend.cpu.pas:1862-1888; cs holds [rows, rot / 2] cos, then
 // sin), K and V stored into the cache at past + row (decoder.pas:
 // 2688-2691); one wave per head
-extern "C" __global__ __launch_bounds__(64) void qkrope(RopeArgs a)
+template <int NV>
+__device__ __forceinline__ void qkrope_t(const RopeArgs& a)
 {
-  // every operand loaded first (heads up to 512: 8 values and 4 rotary
-  // pairs a thread), then the arithmetic: one memory round trip
-  constexpr int NV = 8, NR = 4;
-  __shared__ float nv[512];
-  int hh = blockIdx.x, r = blockIdx.y, t = threadIdx.x;
+  // every operand loaded first (heads of up to 64 NV: NV values and NV / 2
+  // rotary pairs a thread), then the arithmetic: one memory round trip
+  constexpr int NR = NV / 2;
+  __shared__ float nvs[4][64 * NV];
+  float* nv = nvs[threadIdx.x >> 6];
+  const int hh = blockIdx.x, t = threadIdx.x & 63;
+  // a wave past the last row reads it again and stores nothing
+  const int row = blockIdx.y * (blockDim.x >> 6) + (threadIdx.x >> 6), r = min(row, a.rows - 1);
+  const bool live = row < a.rows;
   // (a NoPE layer: no rotating part, every value normed and stored as it is)
   int d = a.hd, half = a.cs ? (a.rot > 0 ? a.rot : d) >> 1 : 0;
   const int past = a.pastp ? *a.pastp : a.past;
@@ -543,6 +553,7 @@ extern "C" __global__ __launch_bounds__(64) void qkrope(RopeArgs a)
       if (t + 64 * i < d) nv[t + 64 * i] = xin[i];
   }
   __syncthreads();
+  if (!live) return;
   int64_t kvw = (int64_t)a.kvh * d;
   int64_t dst = ((int64_t)past + r) * kvw + (int64_t)h * d;
 #pragma unroll
@@ -596,6 +607,13 @@ extern "C" __global__ __launch_bounds__(64) void qkrope(RopeArgs a)
     }
   }
 }
+
+// heads of up to 128, 256 and 512 values; four rows a block for a chunk (a
+// block of one wave per head and row, each lane loading 8 values of heads of
+// 128: 28.5 us for 1024 rows of 32 + 4 heads, 17.9 now)
+extern "C" __global__ __launch_bounds__(256) void qkrope_128(RopeArgs a) { qkrope_t<2>(a); }
+extern "C" __global__ __launch_bounds__(256) void qkrope_256(RopeArgs a) { qkrope_t<4>(a); }
+extern "C" __global__ __launch_bounds__(256) void qkrope_512(RopeArgs a) { qkrope_t<8>(a); }
 
 // --------------------------------------------------------------- attention
 struct AttnArgs {
@@ -2929,56 +2947,65 @@ struct PlanArgs {
 // slot placed by a counter of its expert. A slot's place within its expert
 // changes no output row (each row is its own GEMV/GEMM row), so the counters
 // need no order. One block.
-extern "C" __global__ __launch_bounds__(256) void moe_plan(PlanArgs a)
+// (1024 threads and a scan over the lanes: 22.6 us for 8192 slots of 128
+// experts with 256 threads, of which one added the 256 sums; 8.4 now.)
+extern "C" __global__ __launch_bounds__(1024) void moe_plan(PlanArgs a)
 {
+  constexpr int NT = 1024;
   __shared__ int cnt[4096], off[4096], fill[4096];
-  __shared__ int part[256], ipart[256];
-  __shared__ int ntot;
-  const int t = threadIdx.x, E = a.experts, S = a.slots, CH = a.chunk;
-  for (int e = t; e < E; e += 256) cnt[e] = fill[e] = 0;
+  __shared__ int part[NT / 64], ipart[NT / 64];
+  const int t = threadIdx.x, l = t & 63, w = t >> 6, E = a.experts, S = a.slots, CH = a.chunk;
+  for (int e = t; e < E; e += NT) cnt[e] = fill[e] = 0;
   __syncthreads();
-  for (int s = t; s < S; s += 256) {
+  for (int s = t; s < S; s += NT) {
     const int e = a.ids[s];
     if (e >= 0 && e < E) atomicAdd(&cnt[e], 1);
   }
   __syncthreads();
   // thread t owns experts [e0, e1): its sums, scanned over the threads
-  const int per = (E + 255) / 256, e0 = min(E, t * per), e1 = min(E, e0 + per);
+  const int per = (E + NT - 1) / NT, e0 = min(E, t * per), e1 = min(E, e0 + per);
   int sc = 0, si = 0;
   for (int e = e0; e < e1; e++) {
     sc += cnt[e];
     si += (cnt[e] + CH - 1) / CH;
   }
-  part[t] = sc;
-  ipart[t] = si;
-  __syncthreads();
-  if (t == 0) {
-    int rs = 0, ri = 0;
-    for (int i = 0; i < 256; i++) {
-      const int c = part[i], ci = ipart[i];
-      part[i] = rs;
-      ipart[i] = ri;
-      rs += c;
-      ri += ci;
-    }
-    ntot = ri;
-  }
-  __syncthreads();
-  {
-    int rs = part[t], ri = ipart[t];
-    for (int e = e0; e < e1; e++) {
-      off[e] = rs;
-      for (int st = 0; st < cnt[e]; st += CH)
-        if (ri + st / CH < a.max_items)
-          a.items[ri + st / CH] = make_int4(e, rs + st, min(CH, cnt[e] - st), 0);
-      rs += cnt[e];
-      ri += (cnt[e] + CH - 1) / CH;
+  int rs = sc, ri = si;  // inclusive over the wave, then less the own
+#pragma unroll
+  for (int k = 1; k < 64; k <<= 1) {
+    const int a0 = __shfl_up(rs, k), a1 = __shfl_up(ri, k);
+    if (l >= k) {
+      rs += a0;
+      ri += a1;
     }
   }
+  if (l == 63) {
+    part[w] = rs;
+    ipart[w] = ri;
+  }
+  rs -= sc;
+  ri -= si;
   __syncthreads();
-  for (int s = t; s < S; s += 256) {
+  int ntot = 0;
+#pragma unroll
+  for (int i = 0; i < NT / 64; i++) {
+    if (i < w) {
+      rs += part[i];
+      ri += ipart[i];
+    }
+    ntot += ipart[i];
+  }
+  for (int e = e0; e < e1; e++) {
+    off[e] = rs;
+    for (int st = 0; st < cnt[e]; st += CH)
+      if (ri + st / CH < a.max_items)
+        a.items[ri + st / CH] = make_int4(e, rs + st, min(CH, cnt[e] - st), 0);
+    rs += cnt[e];
+    ri += (cnt[e] + CH - 1) / CH;
+  }
+  __syncthreads();
+  for (int s = t; s < S; s += NT) {
     const int e = a.ids[s];
     if (e >= 0 && e < E) a.perm[off[e] + atomicAdd(&fill[e], 1)] = s;
   }
-  for (int it = ntot + t; it < a.max_items; it += 256) a.items[it] = make_int4(0, 0, 0, 0);
+  for (int it = ntot + t; it < a.max_items; it += NT) a.items[it] = make_int4(0, 0, 0, 0);
 }
