@@ -315,12 +315,27 @@ int enqueue_quantize(ihip_ctx* c, uint64_t x, int64_t rows, int64_t in, int kind
     int* bad;
     int32_t rows, in;
   } a = {(const float*)x, (uint8_t*)xq, (int*)c->scratch_bad, (int32_t)rows, (int32_t)in};
-  if (kind == 0) {
-    int64_t G = in / 32;
-    return launch(c, "quantize_q8_0", dim3((unsigned)((G + 255) / 256), (unsigned)rows), dim3(256), &a);
-  }
+  if (kind == 0)
+    return launch(c, "quantize_q8_0", dim3((unsigned)((in + 1023) / 1024), (unsigned)rows), dim3(256), &a);
   int64_t NB = in / 256;
   return launch(c, "quantize_q8_k", dim3((unsigned)((NB + 3) / 4), (unsigned)rows), dim3(256), &a);
+}
+
+int enqueue_glu_quantize(ihip_ctx* c, uint64_t gate, uint64_t up, int64_t rows, int64_t in, int kind,
+                         uint64_t xq, float alpha, float limit)
+{
+  struct {
+    const float* x;
+    uint8_t* xq;
+    int* bad;
+    int32_t rows, in;
+    const float* up;
+    float alpha, limit;
+  } a = {(const float*)gate, (uint8_t*)xq, (int*)c->scratch_bad, (int32_t)rows, (int32_t)in, (const float*)up,
+         alpha, limit};
+  const int64_t blocks = kind == 0 ? (in + 1023) / 1024 : (in / 256 + 3) / 4;
+  return launch(c, kind == 0 ? "glu_quantize_q8_0" : "glu_quantize_q8_k", dim3((unsigned)blocks, (unsigned)rows),
+                dim3(256), &a);
 }
 
 // weight types of gemm.hip

@@ -218,6 +218,9 @@ bool gemm_runs(const ihip_ctx* c, int dtype, int mode);
 // weights), 0 Q8_0, 1 Q8_K
 int q8_kind(int dtype);
 int enqueue_quantize(ihip_ctx* c, uint64_t x, int64_t rows, int64_t in, int kind, uint64_t xq);
+// the gated activation of gate and up (limit < 0: GeGLU, else SwiGLU) quantized
+int enqueue_glu_quantize(ihip_ctx* c, uint64_t gate, uint64_t up, int64_t rows, int64_t in, int kind,
+                         uint64_t xq, float alpha, float limit);
 // flash-decoding attention: ranges of at most 128 keys per block, then a merge;
 // part holds heads * rows * splits * (hd + 2) doubles; pastp: the position
 // of row 0 in device memory (graph replay), or 0: past

@@ -965,6 +965,13 @@ static int layers(ihip_mctx* s, int64_t n, int64_t past, bool graph)
     }
     return ihip_enqueue_swiglu(m->c, gate, up, count, d.swiglu_alpha, d.swiglu_limit);
   };
+  // a chunk's activation straight into the quantized input of its down
+  // projection (of type dt)
+  auto activate_quant = [&](int dt) { return m->mode == IHIP_MODE_Q8 && q8_kind(dt) >= 0; };
+  auto glu_quantize = [&](int64_t rows, int64_t width, int dt) {
+    return enqueue_glu_quantize(m->c, s->gate, s->up, rows, width, q8_kind(dt), s->xqf, d.swiglu_alpha,
+                                d.activation == IHIP_ACT_GELU_TANH ? -1.0f : std::max(d.swiglu_limit, 0.0f));
+  };
   auto norm = [&](uint64_t x, uint64_t w, uint64_t y) { return ihip_enqueue_rmsnorm(m->c, x, w, y, n, H, d.rms_eps); };
   int rc = norm(s->x, m->L[0].input_norm, s->h);
   if (rc) return rc;
@@ -1035,6 +1042,7 @@ static int layers(ihip_mctx* s, int64_t n, int64_t past, bool graph)
     if (L.moe != IHIP_FFN_MOE) {
       // DenseFfn (decoder.pas:2866-2878)
       const int64_t F = d.ffn;
+      QCache qg{s->xqf, s->xqf};
       if (glu_fused) {
         // gate, up and SwiGLU in one pass
         LinearCall k;
@@ -1046,9 +1054,10 @@ static int layers(ihip_mctx* s, int64_t n, int64_t past, bool graph)
       } else {
         if ((rc = lin(s, s->h, qfp, n, H, L.gd, L.gate, F, 0, s->gate))) return rc;
         if ((rc = lin(s, s->h, qfp, n, H, L.ud, L.up, F, 0, s->up))) return rc;
-        if ((rc = activate(s->gate, s->up, n * F))) return rc;
+        const bool quant = !one && activate_quant(L.dd);
+        if ((rc = quant ? glu_quantize(n, F, L.dd) : activate(s->gate, s->up, n * F))) return rc;
+        (q8_kind(L.dd) == 1 ? qg.havek : qg.have0) = quant;
       }
-      QCache qg{s->xqf, s->xqf};
       if ((rc = lin(s, s->gate, one ? nullptr : &qg, n, F, L.dd, L.down, H, 0, s->tmp))) return rc;
     }
     if (L.moe != IHIP_FFN_DENSE) {
@@ -1156,9 +1165,10 @@ static int layers(ihip_mctx* s, int64_t n, int64_t past, bool graph)
         if ((rc = lin_ids(s, s->h, xqu, n, H, L.eud, L.eu, L.eg_stride, FI, s->ids_dev, n * K, (int)K,
                           L.eub, s->up, qu)))
           return rc;
-        if ((rc = activate(s->gate, s->up, n * K * FI))) return rc;
+        const bool quant = activate_quant(L.edd);
+        if ((rc = quant ? glu_quantize(n * K, FI, L.edd) : activate(s->gate, s->up, n * K * FI))) return rc;
         if ((rc = lin_ids(s, s->gate, s->xqf, n * K, FI, L.edd, L.ed, L.ed_stride, H, s->ids_dev,
-                          n * K, 1, L.edb, s->eout, false)))
+                          n * K, 1, L.edb, s->eout, quant)))
           return rc;
       }
       if (tailed) {
