@@ -150,8 +150,9 @@ __device__ __forceinline__ void quantize_q8_k_t(const A& args)
 extern "C" __global__ __launch_bounds__(256) void quantize_q8_0(QuantArgs a) { quantize_q8_0_t<false>(a); }
 extern "C" __global__ __launch_bounds__(256) void quantize_q8_k(QuantArgs a) { quantize_q8_k_t<false>(a); }
 // a prompt chunk's activation into the down projection's input: the gated
-// values are not written and read as floats in between (8192 rows of 768 in
-// two MoE layers: 2 x (16.8 + 9) us as two launches, GLUQ_US)
+// values are not written and read as floats in between (8192 rows of 768 to
+// Q8_K 16.8 and 9 us as two launches, 20.5 as one; 512 rows of 3584 to Q8_0
+// 5.6 and 4.2, 6.5 as one)
 extern "C" __global__ __launch_bounds__(256) void glu_quantize_q8_0(GluQuantArgs a) { quantize_q8_0_t<true>(a); }
 extern "C" __global__ __launch_bounds__(256) void glu_quantize_q8_k(GluQuantArgs a) { quantize_q8_k_t<true>(a); }
 
