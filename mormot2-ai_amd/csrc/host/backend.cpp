@@ -476,10 +476,12 @@ int enqueue_linear(ihip_ctx* c, const LinearCall& k)
   // GEMM's first 32 rows cost one tile (BF16, us, launches / GEMM: 4 rows of
   // 2048 -> 6144 38.9 / 30.1, 2 rows 21 / 30; 8 rows of 3072 -> 1024 29.9 /
   // 24.8, of 1024 -> 3072 22.2 / 19.5, of 2048 -> 512 13.0 / 18.5; 4 rows of
-  // 1024 -> 40000 94.8 / 90.9)
+  // 1024 -> 40000 94.8 / 90.9; where the GEMM may not split its sum, those
+  // few blocks walk it whole: left to the launches)
   const int64_t elems = k.in * k.out;
   const bool few = q8 ? c->gemm_few_rows && k.rows > 8 && (k.rows + 7) / 8 * k.out >= 6144
-                      : c->gemm_few_float && (k.rows >= 4 && elems >= 12 << 20 || k.rows >= 8 && elems >= 3 << 20);
+                      : c->gemm_few_float && !k.no_alloc && !c->capturing &&
+                        (k.rows >= 4 && elems >= 12 << 20 || k.rows >= 8 && elems >= 3 << 20);
   if (batch && gemm_q8 && (k.items ? k.item_rows > 8 : k.rows >= min_rows || few)) {
     struct {
       const uint8_t* w;

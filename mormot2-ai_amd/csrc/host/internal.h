@@ -82,7 +82,7 @@ struct ihip_ctx {
   int gemm_min_rows_float = ihip::GEMM_MIN_ROWS_FLOAT;
   int gemv_blocks_per_cu = 2;  // one-row GEMV launches: blocks per CU at least (IHIP_GEMV_BLOCKS_PER_CU)
   int gemv_hold = 1;  // one-row GEMV launches: at most this many rounds of resident blocks (IHIP_GEMV_HOLD)
-  bool use_gemm8 = true;  // 2..79 quantized rows on the int8 matrix cores, gemm8 (IHIP_GEMM8=0: the VALU gemv_rows)
+  bool use_gemm8 = true;  // the quantized rows gemm does not take on the int8 matrix cores, gemm8 (IHIP_GEMM8=0: the VALU gemv_rows)
   // MXFP4 prefill GEMMs on the scaled f8f6f4 matrix cores (IHIP_GEMM_F8=1)
   // rather than the int8 ones
   bool gemm_f8 = false;
