@@ -1128,6 +1128,12 @@ extern "C" __global__ __launch_bounds__(256) void attention_rows_f32_128(AttnArg
 // (the values), so each lane reads its own contiguous part of a row: the sum
 // is over the same terms, permuted.
 //
+// A key that a row of the tile does not see has weight 0 in it, and its value
+// meets that weight in the product: 0 only while it is finite, else a NaN. So a
+// block whose sums are not all finite forms them again (`odd`): its products then
+// leave out the values that are not finite, and each row that sees such a
+// value's key adds it on its own.
+//
 // Bound by the f64 matrix cores (4 hd operations a row and key, a 64-cycle
 // MFMA per 2048: 111 of the 188 us below) and the vector instructions beside
 // them, which the counters show in sequence with them rather than under them:
@@ -1176,6 +1182,7 @@ __device__ __forceinline__ void attention_mfma_t(const AttnArgs& a)
   __shared__ double sc[2][ATTM][ATTMK + 1];  // scores, then weights (row, key of the range)
   __shared__ double stat[ATTM][2];           // a row's running maximum and sum
   __shared__ double shrink[ATTM];            // exp(old maximum - new maximum)
+  __shared__ int odds[4];                    // a wave holds a sum that is not finite
   const int h = xcd_head(blockIdx.x, a.heads), s = blockIdx.z;
   // the tiles with the most keys first
   const int r0 = (int)(gridDim.y - 1 - blockIdx.y) * ATTM;
@@ -1195,10 +1202,6 @@ __device__ __forceinline__ void attention_mfma_t(const AttnArgs& a)
   const int per = span <= ATTMK ? ATTMK : ATT_CHUNK;
   const int nit = (span + per - 1) / per;
   const int it0 = s * nit / a.splits, it1 = (s + 1) * nit / a.splits;
-  if (t < ATTM) {
-    stat[t][0] = -1.0e308;
-    stat[t][1] = 0.0;
-  }
   constexpr int DQ = d / 4;  // scores: k steps = a lane's dimensions
   float qa[DQ];  // (widened at each use: as doubles they halve the waves a SIMD holds)
   {
@@ -1214,8 +1217,15 @@ __device__ __forceinline__ void attention_mfma_t(const AttnArgs& a)
     }
   }
   constexpr int NT = d / 64;  // values: dimensions of a lane, one per tile
+  constexpr uint32_t ES = F16 ? 2 : 4;
   const int dim0 = w * (d / 4) + NT * lc;
   dbl4 o[NT];
+  bool odd = false;
+again:
+  if (t < ATTM) {
+    stat[t][0] = -1.0e308;
+    stat[t][1] = 0.0;
+  }
 #pragma unroll
   for (int n = 0; n < NT; n++) o[n] = dbl4{0.0, 0.0, 0.0, 0.0};
   __syncthreads();
@@ -1279,7 +1289,8 @@ __device__ __forceinline__ void attention_mfma_t(const AttnArgs& a)
 #pragma unroll
       for (int i = 0; i < NB; i++)
         if (i < nblk) {
-          const double y = x[i] > -1.0e308 ? exp_below(x[i] - m) : 0.0;
+          // (a NaN score stays one, as in the CPU's sum)
+          const double y = x[i] == -1.0e308 ? 0.0 : exp_below(x[i] - m);
           pr[16 * i] = y;
           e += y;
         }
@@ -1305,46 +1316,54 @@ __device__ __forceinline__ void attention_mfma_t(const AttnArgs& a)
     }
     const int S = nk >> 2;  // k steps (nk is a multiple of 16)
     constexpr int VU = NT > 2 ? 4 : 12;  // value loads in flight per lane
-    constexpr uint32_t ES = F16 ? 2 : 4;
     // a uniform base and 24-bit products for the lane's offset (a range is at
     // most ATTMK rows of kvw values)
     const uint8_t* vbase = (const uint8_t*)a.vc + ((int64_t)kb * kvw + (int64_t)g * d) * ES;
     const uint32_t vlast = (uint32_t)(ke - 1 - kb), vrow = (uint32_t)kvw * ES, vdim = (uint32_t)dim0 * ES;
+    // this lane's values of key k of the range (past the last: the last)
+    auto values = [&](uint32_t k, float (&v)[NT]) __attribute__((always_inline)) {
+      const uint8_t* vp = vbase + (__umul24(min(k, vlast), vrow) + vdim);
+      if constexpr (F16) {
+        if constexpr (NT == 1) {
+          v[0] = half_to_float(*(const uint16_t*)vp);
+        } else {
+          uint32_t x[NT / 2];
+          if constexpr (NT == 2) {
+            x[0] = *(const uint32_t*)vp;
+          } else {
+            const uint2 y = *(const uint2*)vp;
+            x[0] = y.x;
+            x[1] = y.y;
+          }
+#pragma unroll
+          for (int n = 0; n < NT; n++) v[n] = half_to_float((n & 1) ? x[n / 2] >> 16 : x[n / 2] & 0xffffu);
+        }
+      } else {
+        if constexpr (NT == 1) {
+          v[0] = *(const float*)vp;
+        } else if constexpr (NT == 2) {
+          const float2 x = *(const float2*)vp;
+          v[0] = x.x;
+          v[1] = x.y;
+        } else {
+          const float4 x = *(const float4*)vp;
+          v[0] = x.x;
+          v[1] = x.y;
+          v[2] = x.z;
+          v[3] = x.w;
+        }
+      }
+    };
+    auto finite = [](float v) __attribute__((always_inline)) { return (float_bits(v) & 0x7f800000u) != 0x7f800000u; };
     for (int t0 = 0; t0 < S; t0 += VU) {
       float vv[VU][NT];
 #pragma unroll
-      for (int u = 0; u < VU; u++) {
-        const uint8_t* vp = vbase + (__umul24(min((uint32_t)(lq * S + t0 + u), vlast), vrow) + vdim);
-        if constexpr (F16) {
-          if constexpr (NT == 1) {
-            vv[u][0] = half_to_float(*(const uint16_t*)vp);
-          } else {
-            uint32_t x[NT / 2];
-            if constexpr (NT == 2) {
-              x[0] = *(const uint32_t*)vp;
-            } else {
-              const uint2 y = *(const uint2*)vp;
-              x[0] = y.x;
-              x[1] = y.y;
-            }
+      for (int u = 0; u < VU; u++) values(lq * S + t0 + u, vv[u]);
+      if (odd) {
 #pragma unroll
-            for (int n = 0; n < NT; n++) vv[u][n] = half_to_float((n & 1) ? x[n / 2] >> 16 : x[n / 2] & 0xffffu);
-          }
-        } else {
-          if constexpr (NT == 1) {
-            vv[u][0] = *(const float*)vp;
-          } else if constexpr (NT == 2) {
-            const float2 x = *(const float2*)vp;
-            vv[u][0] = x.x;
-            vv[u][1] = x.y;
-          } else {
-            const float4 x = *(const float4*)vp;
-            vv[u][0] = x.x;
-            vv[u][1] = x.y;
-            vv[u][2] = x.z;
-            vv[u][3] = x.w;
-          }
-        }
+        for (int u = 0; u < VU; u++)
+#pragma unroll
+          for (int n = 0; n < NT; n++) vv[u][n] = finite(vv[u][n]) ? vv[u][n] : 0.f;
       }
 #pragma unroll
       for (int u = 0; u < VU; u++) {
@@ -1356,9 +1375,38 @@ __device__ __forceinline__ void attention_mfma_t(const AttnArgs& a)
         }
       }
     }
+    if (odd) {
+      for (int k = 0; k < ke - kb; k++) {
+        float x[NT];
+        values(k, x);
+#pragma unroll
+        for (int n = 0; n < NT; n++)
+          if (!finite(x[n]))
+#pragma unroll
+            for (int v = 0; v < 4; v++) {
+              const int r = lq + 4 * v;
+              if (kb + k >= first(r) && kb + k <= past + r0 + r) o[n][v] = __builtin_fma(p[r][k], (double)x[n], o[n][v]);
+            }
+      }
+    }
+  }
+  if (!odd) {
+    bool bad = false;
+#pragma unroll
+    for (int n = 0; n < NT; n++)
+#pragma unroll
+      for (int v = 0; v < 4; v++) bad |= !(fabs(o[n][v]) <= 1.7976931348623157e308);
+    const bool any = __any(bad);
+    if (l == 0) odds[w] = any;
+    __syncthreads();
+    if (odds[0] | odds[1] | odds[2] | odds[3]) {
+      odd = true;
+      goto again;
+    }
   }
   // ---- row lq + 4 v, dimension(s) dim0 + n: the output, or the partial sums
-  // with the row's maximum and sum (an empty group: weight 0 in the merge)
+  // with the row's maximum and sum (an empty group's: -1e308 and 0, weight 0 in
+  // the merge)
 #pragma unroll
   for (int v = 0; v < 4; v++) {
     const int r = lq + 4 * v;
@@ -1368,9 +1416,8 @@ __device__ __forceinline__ void attention_mfma_t(const AttnArgs& a)
 #pragma unroll
       for (int n = 0; n < NT; n++) out[dim0 + n] = o[n][v];
       if (w == 0 && lc == 0) {
-        const bool empty = !(stat[r][1] > 0.0);
-        out[d] = empty ? -1.0e308 : stat[r][0];
-        out[d + 1] = empty ? 0.0 : stat[r][1];
+        out[d] = stat[r][0];
+        out[d + 1] = stat[r][1];
       }
       continue;
     }
