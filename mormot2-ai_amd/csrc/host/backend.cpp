@@ -552,10 +552,18 @@ int enqueue_linear(ihip_ctx* c, const LinearCall& k)
     if (float_fmt(k.dtype)) return launch(c, gname, dim3(gx, gy), dim3(256), &g);
     // blocks of 32 MT rows x 128 / KS outputs: from four 32 x 128 tiles a CU
     // a K-quant takes 64 rows (its decode shared); with fewer than two a CU
-    // the waves of a block share the sum, in 2 parts, then in 4
+    // the waves of a block share the sum, in 2 parts, then in 4, as far as it
+    // has chunks of 256 values for them: a part without one leaves its wave
+    // idle in every block, so the fuller the chip, the more chunks a part
+    // needs (KS 1 / 2 / 4, us, medians over the block types: 72 rows of 256 ->
+    // 6144 7.2 / 7.7 / 12.1; 300 of 512 -> 2048 9.3 / 9.2 / 13.1, of 1024 -> 2048
+    // 13.4 / 12.8 / 13.6, of 2048 -> 1024 22.1 / 14.1 / 13.8)
     const int64_t tiles32 = (k.items ? 2 * k.nitems : (k.rows + 31) / 32) * ((k.out + 127) / 128);
     const bool wide = q8_kind(k.dtype) == 1 && (k.items || tiles32 >= 4 * (int64_t)c->cus);
-    const int ks = k.items || tiles32 >= 2 * (int64_t)c->cus ? 1 : 4 * tiles32 >= 3 * (int64_t)c->cus ? 2 : 4;
+    const int64_t nch = (G + 7) / 8, cus = c->cus;
+    int ks = 1;
+    if (!k.items && ((tiles32 < 2 * cus && nch >= 4) || (4 * tiles32 < 3 * cus && nch >= 2))) ks = 2;
+    if (!k.items && ((4 * tiles32 < 3 * cus && nch >= 6) || (8 * tiles32 < 3 * cus && nch >= 3))) ks = 4;
     snprintf(gname, sizeof gname, "gemm_%s_m%dk%d", fmt_name(k.dtype), wide ? 2 : 1, ks);
     const unsigned by = (unsigned)(k.items ? (wide ? 1 : 2) * k.nitems : (k.rows + (wide ? 63 : 31)) / (wide ? 64 : 32));
     const int64_t bn = 128 / ks;

@@ -51,6 +51,37 @@ def test_tiles_match_oracle(ctx, dtype):
         assert (bits > 0).mean() <= 1e-3
 
 
+def same(got, ref):
+    """At most one ulp of single apart, in at most 1/1000 of the values."""
+    bits = np.abs(got.view(np.int32).astype(np.int64) - ref.view(np.int32).astype(np.int64))
+    # (a value within a rounding of zero may change its sign bit: compared by size)
+    near = np.abs(got - ref) <= np.abs(ref) * 2.0 ** -23 + 1e-30
+    assert np.all((bits <= 1) | near), int(bits.max())
+    assert (bits > 0).mean() <= 1e-3
+
+
+# (rows, in, out, the parts of the sum on 256 CUs): by the 32 x 128 tiles and
+# the sum's chunks of 256 values, no part without a chunk
+PARTS = [(72, 256, 6144, 1), (97, 256, 130, 1), (300, 512, 2048, 2), (100, 512, 700, 2), (200, 768, 700, 4),
+         (200, 768, 3072, 2), (200, 768, 3500, 1), (300, 1024, 2048, 2), (300, 1280, 2048, 2),
+         (300, 1536, 2048, 4), (300, 2048, 1024, 4), (200, 2048, 3500, 2), (520, 1024, 4000, 1)]
+
+
+@pytest.mark.parametrize("rows,cols,out,parts", PARTS)
+def test_parts_of_the_sum(ctx, rows, cols, out, parts):
+    if ctx.info()[2] != 256:
+        pytest.skip("the line lies at other sizes on another number of CUs")
+    x = np.random.default_rng(rows + out).standard_normal((rows, cols)).astype(np.float32)
+    for dtype in (H.Q4_0, H.Q6_K):
+        w = H.synth_blocks(dtype, out, cols, rows + cols, -8, -4)
+        ctx.kernel_timer("gemm", 16)
+        got = ctx.linear(x, w, dtype, out, mode=H.MODE_Q8)
+        names = list(ctx.kernel_timer_report())
+        ctx.kernel_timer(None)
+        assert names == ["gemm_%s_m1k%d" % (H.NAMES[dtype].lower(), parts)]
+        same(got, O.linear(x, w, dtype, out, None))
+
+
 def test_quantized_input_and_rows_apart(ctx):
     # a row's result does not depend on the rows beside it, nor on who
     # quantized it
