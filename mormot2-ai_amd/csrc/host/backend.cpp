@@ -465,23 +465,30 @@ int enqueue_linear(ihip_ctx* c, const LinearCall& k)
   if (k.items && k.item_rows > 8 && !gemm_q8)
     return fail(IHIP_E_ARG, "EnqueueLinear: items of more than 8 slots need the GEMM");
   const int min_rows = float_fmt(k.dtype) ? c->gemm_min_rows_float : c->gemm_min_rows;
-  // quantized weights, fewer rows than that: the 8-row launches below take
-  // about 5.5 us and 10 us per 10^6 (8 rows, output, group)s, the GEMM 5 us
-  // and 2 us per 1024 values of the sum, so the GEMM wins from about
-  // 6144 (8 rows, output)s whatever the sum's length (Q4_K, us, 8-row
-  // launches / GEMM: 16 rows of 2048 -> 6144 13.8 / 8.4, 16 of 1024 -> 3072
-  // 7.5 / 6.9, 48 of 3072 -> 1024 10.9 / 10.9, 32 of it 9.5 / 11.0, 64 of
-  // 2048 -> 512 8.2 / 9.2, 16 of 1024 -> 40000 20.4 / 11.3)
+  // quantized weights, fewer rows than that: the 8-row launches' time grows
+  // with the (8 rows, output, group)s, the GEMM's with the chunks of a part of
+  // the sum, and it needs enough (8 rows, output)s to fill the chip. The lines
+  // are the lowest at which none of 7 types x 9 sums of 256 .. 8192 x 12 output
+  // counts x 13 row counts runs over 6% slower than the 8-row launches, but one
+  // Q8_0 shape (12%); Q6_K's two products a group and Q5_1's second term pay
+  // later (us, 8-row launches / GEMM: 16 rows of 2048 -> 6144 Q4_K 14.3 / 8.8, Q6_K
+  // 14.9 / 10.1; 24 of 8192 -> 2048 Q4_K 49.3 / 21.0; left to the launches: 9 of 2048 ->
+  // 3072 Q5_1 9.5 / 11.3, 9 of 2048 -> 4096 Q8_0 8.0 / 10.0, 17 of 2048 -> 2048 Q6_K
+  // 8.1 / 10.0)
   // float weights: the 8-row launches' time grows with rows x weights, the
   // GEMM's first 32 rows cost one tile (BF16, us, launches / GEMM: 4 rows of
   // 2048 -> 6144 38.9 / 30.1, 2 rows 21 / 30; 8 rows of 3072 -> 1024 29.9 /
   // 24.8, of 1024 -> 3072 22.2 / 19.5, of 2048 -> 512 13.0 / 18.5; 4 rows of
-  // 1024 -> 40000 94.8 / 90.9; where the GEMM may not split its sum, those
-  // few blocks walk it whole: left to the launches)
-  const int64_t elems = k.in * k.out;
-  const bool few = q8 ? c->gemm_few_rows && k.rows > 8 && (k.rows + 7) / 8 * k.out >= 6144
-                      : c->gemm_few_float && !k.no_alloc && !c->capturing &&
-                        (k.rows >= 4 && elems >= 12 << 20 || k.rows >= 8 && elems >= 3 << 20);
+  // 1024 -> 40000 94.8 / 90.9; F32 and F16 lie the same way on both sides of
+  // the lines; where the GEMM may not split its sum, those few blocks walk it
+  // whole: left to the launches)
+  const int64_t elems = k.in * k.out, outs8 = (k.rows + 7) / 8 * k.out;
+  const bool few =
+      q8 ? c->gemm_few_rows && k.rows > 8 &&
+               ((outs8 >= 9216 && outs8 * G >= (k.dtype == DT_Q6_K || k.dtype == DT_Q5_1 ? 500000 : 400000)) ||
+                (outs8 >= 6144 && outs8 * G >= 1500000 && k.dtype != DT_Q5_1))
+         : c->gemm_few_float && !k.no_alloc && !c->capturing &&
+               ((k.rows >= 4 && elems >= 12 << 20) || (k.rows >= 8 && elems >= 3 << 20));
   if (batch && gemm_q8 && (k.items ? k.item_rows > 8 : k.rows >= min_rows || few)) {
     struct {
       const uint8_t* w;

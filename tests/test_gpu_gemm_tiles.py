@@ -62,7 +62,7 @@ def same(got, ref):
 
 # (rows, in, out, the parts of the sum on 256 CUs): by the 32 x 128 tiles and
 # the sum's chunks of 256 values, no part without a chunk
-PARTS = [(72, 256, 6144, 1), (97, 256, 130, 1), (300, 512, 2048, 2), (100, 512, 700, 2), (200, 768, 700, 4),
+PARTS = [(80, 256, 6144, 1), (97, 256, 130, 1), (300, 512, 2048, 2), (100, 512, 700, 2), (200, 768, 700, 4),
          (200, 768, 3072, 2), (200, 768, 3500, 1), (300, 1024, 2048, 2), (300, 1280, 2048, 2),
          (300, 1536, 2048, 4), (300, 2048, 1024, 4), (200, 2048, 3500, 2), (520, 1024, 4000, 1)]
 
@@ -80,6 +80,27 @@ def test_parts_of_the_sum(ctx, rows, cols, out, parts):
         ctx.kernel_timer(None)
         assert names == ["gemm_%s_m1k%d" % (H.NAMES[dtype].lower(), parts)]
         same(got, O.linear(x, w, dtype, out, None))
+
+
+# (type, rows, in, out, on the GEMM): 9 to 79 rows on either side of the line
+# to the 8-row launches, which depends on the sum's length and the type
+SHORT = [(H.Q4_K, 16, 2048, 6144, True), (H.Q6_K, 16, 2048, 6144, True), (H.Q4_K, 9, 2048, 4608, True),
+         (H.Q5_1, 9, 2048, 3072, False), (H.Q8_0, 9, 2048, 4096, False), (H.Q6_K, 17, 2048, 2048, False),
+         (H.MXFP4, 9, 768, 8192, False), (H.Q4_0, 24, 8192, 2048, True), (H.Q5_1, 24, 8192, 2048, False),
+         (H.Q6_K, 33, 1280, 2048, False), (H.Q5_0, 79, 1024, 1300, True), (H.Q4_0, 8, 2048, 8192, False),
+         (H.Q8_0, 33, 512, 3000, False), (H.Q6_K, 40, 2048, 1700, False)]
+
+
+@pytest.mark.parametrize("dtype,rows,cols,out,gemm", SHORT)
+def test_short_batches(ctx, dtype, rows, cols, out, gemm):
+    x = np.random.default_rng(rows + out).standard_normal((rows, cols)).astype(np.float32)
+    w = H.synth_blocks(dtype, out, cols, rows + cols, -8, -4)
+    ctx.kernel_timer("ge", 16)
+    got = ctx.linear(x, w, dtype, out, mode=H.MODE_Q8)
+    names = list(ctx.kernel_timer_report())
+    ctx.kernel_timer(None)
+    assert len(names) == 1 and names[0].startswith("gemm_") == gemm, names
+    same(got, O.linear(x, w, dtype, out, None))
 
 
 def test_quantized_input_and_rows_apart(ctx):
