@@ -1286,6 +1286,21 @@ int enqueue_attention_one(ihip_ctx* c, const AttnOne& o)
   return launch(c, "attention_merge", dim3((unsigned)o.heads, 1), dim3(128), &mg);
 }
 
+// the groups that the key ranges of `tiles` (head, 16 rows) tiles are shared
+// between, each a block: one, with no merge, where the tiles give every CU two
+// blocks or there are two ranges at most and enough rows that the merge costs
+// more than a block's second range (32 heads of 128, 100 rows after 60: 25.5 us in two
+// groups, 13.4 in one); else as many as give every CU two, or one more where the
+// fullest CU then walks fewer ranges (16 heads of 128, 100 rows after 2000: 112 tiles, 17
+// ranges: 5 groups 75.2 us, 6 groups 63.8)
+static int attention_groups(int64_t tiles, int64_t heads, int64_t rows, int64_t splits, int64_t cus)
+{
+  if (tiles >= 2 * cus || (splits <= 2 && heads * rows >= 4 * cus)) return 1;
+  const auto ranges = [&](int64_t g) { return (tiles * g + cus - 1) / cus * ((splits + g - 1) / g); };
+  const int64_t g = std::min(splits, (2 * cus + tiles - 1) / tiles);
+  return (int)(g < splits && 2 * tiles * (g + 1) <= 7 * cus && ranges(g + 1) < ranges(g) ? g + 1 : g);
+}
+
 int enqueue_attention(ihip_ctx* c, uint64_t q, uint64_t kc, uint64_t vc, uint64_t y, uint64_t part,
                       int64_t rows, int64_t heads, int64_t kvh, int64_t hd, int64_t past,
                       uint64_t pastp, int64_t window, uint64_t sinks, double scale, int f16,
@@ -1307,13 +1322,19 @@ int enqueue_attention(ihip_ctx* c, uint64_t q, uint64_t kc, uint64_t vc, uint64_
          (const int*)pastp, (double*)part, scale, (int32_t)rows, (int32_t)heads, (int32_t)kvh,
          (int32_t)hd, (int32_t)past, (int32_t)window, f16, splits};
   int rc;
-  if ((hd == 64 || hd == 128 || hd == 256) && rows > 1 && c->attn_mfma && kvh * hd < 1 << 22) {
-    // tiles of 16 rows on the f64 matrix cores, a block per tile and head when
-    // these give every CU two, else the tile's key ranges in as many groups
-    // (with a merge) as do; the offsets inside a range are 24-bit products
+  // few rows of half-float heads of 256: a block of the tiles below walks 16
+  // rows of a range however few there are, 19 us at best, where attention_part's
+  // blocks, one per row and range, take 16 while they fit in one or two rounds
+  // (8 heads: 8 rows after 500 16.5 us there, 19.9 in tiles; 8 rows after 2000 in a window
+  // of 1024 19.9, 24.3; 32 rows after 500 29.3, 21.4; float keys are slower there at once)
+  const int64_t keys = window > 0 ? std::min(past + rows, window) : past + rows, blocks = heads * rows * splits;
+  const bool few = hd == 256 && f16 &&
+                   (splits == 1 ? keys >= 72 && blocks <= c->cus : 2 * blocks <= (splits <= 8 ? 5 : 4) * c->cus);
+  if ((hd == 64 || hd == 128 || hd == 256) && rows > 1 && c->attn_mfma && kvh * hd < 1 << 22 && !few) {
+    // tiles of 16 rows on the f64 matrix cores, a block per tile, head and group
+    // of the tile's key ranges; the offsets inside a range are 24-bit products
     // of its rows' bytes
-    const int64_t tiles = heads * ((rows + 15) / 16);
-    const int groups = (int)std::min<int64_t>(splits, tiles >= 2 * c->cus ? 1 : (2 * c->cus + tiles - 1) / tiles);
+    const int groups = attention_groups(heads * ((rows + 15) / 16), heads, rows, splits, c->cus);
     a.splits = groups;
     char name[32];
     snprintf(name, sizeof name, "attention_mfma_%s_%d", f16 ? "f16" : "f32", (int)hd);

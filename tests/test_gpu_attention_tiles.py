@@ -56,6 +56,29 @@ def test_tiles_match_oracle(ctx, heads, kvh, hd, rows, past, window, sinks, half
     assert np.abs(got - ref).max() <= 2e-7 * np.abs(ref).max()
 
 
+# heads, kv heads, head size, rows, past, window, half, and the kernels that run:
+# tiles with and without a merge, rows on their own (few rows of half-float heads
+# of 256)
+ROUTES = [
+    (32, 4, 128, 100, 60, 0, True, "mfma"), (14, 2, 64, 200, 0, 0, False, "mfma"),
+    (8, 2, 128, 100, 60, 0, True, "mfma merge"), (16, 8, 128, 100, 2000, 0, True, "mfma merge"),
+    (14, 2, 64, 300, 2000, 0, True, "mfma merge"), (8, 2, 256, 8, 500, 0, True, "part merge"),
+    (8, 2, 256, 8, 500, 0, False, "mfma merge"), (8, 2, 256, 8, 2000, 1024, True, "part merge"),
+    (8, 2, 256, 16, 2000, 128, True, "part merge"), (8, 2, 256, 64, 60, 0, True, "mfma"),
+    (16, 8, 256, 20, 500, 0, True, "mfma merge"), (8, 2, 256, 9, 0, 0, True, "mfma")]
+
+
+@pytest.mark.parametrize("heads,kvh,hd,rows,past,window,half,names", ROUTES)
+def test_routes_match_oracle(ctx, heads, kvh, hd, rows, past, window, half, names):
+    if ctx.info()[2] != 256:
+        pytest.skip("the lines lie at other sizes on another number of CUs")
+    ctx.kernel_timer("attention_", 16)
+    test_tiles_match_oracle(ctx, heads, kvh, hd, rows, past, window, False, half)
+    got = [k.split("_")[1] for k in ctx.kernel_timer_report()]
+    ctx.kernel_timer(None)
+    assert " ".join(got) == names
+
+
 # heads, kv heads, head size, rows, past, window, sinks, half, and where: the
 # key rows that hold infinities or a NaN (of the total), in the values or keys
 ODD = [
