@@ -103,9 +103,49 @@ def test_short_batches(ctx, dtype, rows, cols, out, gemm):
     same(got, O.linear(x, w, dtype, out, None))
 
 
+@pytest.mark.parametrize("dtype", BLOCK[:5], ids=[H.NAMES[t] for t in BLOCK[:5]])
+@pytest.mark.parametrize("rows", [16, 96])
+def test_subnormal_scales(ctx, dtype, rows):
+    """The products of a row's and a weight's scale are formed from halves on the
+    matrix cores: scales below the least normal half (activations below
+    0.0078, MXFP4 exponents up to 112) keep every bit."""
+    cols, out = 1024, 9000
+    rng = np.random.default_rng(dtype)
+    x = rng.standard_normal((rows, cols)).astype(np.float32)
+    x *= 10.0 ** -rng.uniform(1, 6.5, (rows, cols // 32)).astype(np.float32).repeat(32, 1)
+    bv, bs = H.BLOCK[dtype]
+    b = rng.integers(0, 256, (out, cols // bv, bs), dtype=np.uint8)
+    if dtype == H.MXFP4:
+        b[..., 0] = rng.integers(104, 114, b.shape[:2])
+    else:
+        for i in range(0, 4 if dtype == H.Q5_1 else 2, 2):
+            b[..., i:i + 2] = rng.integers(1, 2048, b.shape[:2]).astype(np.uint16)[..., None].view(np.uint8)
+    w = b.reshape(-1)
+    ctx.kernel_timer("ge", 16)
+    got = ctx.linear(x, w, dtype, out, mode=H.MODE_Q8)
+    names = list(ctx.kernel_timer_report())
+    ctx.kernel_timer(None)
+    assert len(names) == 1 and names[0].startswith("gemm_"), names
+    ref = O.linear(x, w, dtype, out)
+    assert np.count_nonzero(ref) > 0.9 * ref.size
+    same(got, ref)
+
+
+@pytest.mark.parametrize("dtype", [H.Q4_K, H.Q8_0, H.F32], ids=["Q4_K", "Q8_0", "F32"])
+def test_rows_beside_others(ctx, dtype):
+    # the rows beside a row choose the tiles and the parts of its sum (here 4
+    # for the 32 rows alone, 1 among 600), which changes the order of a double sum
+    # and no more
+    rows, cols, out = 600, 2048, 5000
+    x = np.random.default_rng(7).standard_normal((rows, cols)).astype(np.float32)
+    w = H.synth_normal(dtype, out, cols, 5, 0.5) if dtype == H.F32 else H.synth_blocks(dtype, out, cols, 5, -8, -4)
+    whole = ctx.linear(x, w, dtype, out, mode=H.MODE_Q8)
+    same(ctx.linear(x[64:96], w, dtype, out, mode=H.MODE_Q8), whole[64:96])
+
+
 def test_quantized_input_and_rows_apart(ctx):
-    # a row's result does not depend on the rows beside it, nor on who
-    # quantized it
+    # a row's result does not depend on who quantized it, nor on the rows beside
+    # it while they leave the parts of its sum alone
     rows, cols, out = 75, 1024, 2500
     x = np.random.default_rng(3).standard_normal((rows, cols)).astype(np.float32)
     w = H.synth_blocks(H.Q4_K, out, cols, 5, -8, -4)
