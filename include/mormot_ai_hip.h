@@ -54,7 +54,8 @@ enum {
 enum { IHIP_MODE_F32 = 0, IHIP_MODE_Q8 = 1 };
 /* or'ed into IHIP_MODE_Q8: x is a buffer already quantized by
  * ihip_enqueue_quantize (the quantization of a row shared by several
- * Linears is then done once) */
+ * Linears is then done once; its Q8_0 scales are half-float values widened
+ * to single, which the kernels of many rows take as halves) */
 enum { IHIP_MODE_XQ = 2 };
 
 /* ---- status codes ---- */
@@ -176,7 +177,9 @@ int ihip_enqueue_linear_at(ihip_ctx* ctx, uint64_t x, int64_t rows, int64_t in,
  * orders its own calls, so the first context to make a multi-row call holds
  * the array until it is destroyed and a multi-row call of another context on
  * that GPU is refused (IHIP_E_ARG, nothing enqueued). One-row calls use no
- * array. Same arguments and results as ihip_enqueue_linear_at. */
+ * array. Same arguments and results as ihip_enqueue_linear_at; of float
+ * weights of several rows, whose sum may be split only where its parts can be
+ * allocated, up to the order of a double sum. */
 #define IHIP_STATIC_SCRATCH_BYTES (8u << 20)
 int ihip_enqueue_linear_at_static(ihip_ctx* ctx, uint64_t x, int64_t rows, int64_t in,
                                   int dtype, uint64_t w, int64_t out, uint64_t y,

@@ -480,14 +480,25 @@ int enqueue_linear(ihip_ctx* c, const LinearCall& k)
   // 2048 -> 6144 38.9 / 30.1, 2 rows 21 / 30; 8 rows of 3072 -> 1024 29.9 /
   // 24.8, of 1024 -> 3072 22.2 / 19.5, of 2048 -> 512 13.0 / 18.5; 4 rows of
   // 1024 -> 40000 94.8 / 90.9; F32 and F16 lie the same way on both sides of
-  // the lines; where the GEMM may not split its sum, those few blocks walk it
-  // whole: left to the launches)
+  // the lines; where a call may not allocate the parts of a sum that the GEMM
+  // would split, those few blocks walk it whole: left to the launches)
+  const bool flt32 = float_fmt(k.dtype) && !k.items && k.rows <= 32, may_split = !k.no_alloc && !c->capturing;
+  const int64_t bm = flt32 ? 32 : 64;  // rows of a float tile, 4096 / bm outputs
+  // float weights with too few tiles to fill the chip (a router: 128
+  // outputs): the sum split into parts of >= 256 values, one block each, then
+  // their double sums added in split order
+  int flt_parts = 1;
+  if (float_fmt(k.dtype) && !k.items && c->gemm_split) {
+    const int64_t tiles = (k.out + 4096 / bm - 1) / (4096 / bm) * ((k.rows + bm - 1) / bm);
+    while (flt_parts < 16 && tiles * flt_parts * 2 <= (int64_t)c->cus * 2 && k.in / (flt_parts * 2) >= 256)
+      flt_parts *= 2;
+  }
   const int64_t elems = k.in * k.out, outs8 = (k.rows + 7) / 8 * k.out;
   const bool few =
       q8 ? c->gemm_few_rows && k.rows > 8 &&
                ((outs8 >= 9216 && outs8 * G >= (k.dtype == DT_Q6_K || k.dtype == DT_Q5_1 ? 500000 : 400000)) ||
                 (outs8 >= 6144 && outs8 * G >= 1500000 && k.dtype != DT_Q5_1))
-         : c->gemm_few_float && !k.no_alloc && !c->capturing &&
+         : c->gemm_few_float && (may_split || flt_parts == 1) &&
                ((k.rows >= 4 && elems >= 12 << 20) || (k.rows >= 8 && elems >= 3 << 20));
   if (batch && gemm_q8 && (k.items ? k.item_rows > 8 : k.rows >= min_rows || few)) {
     struct {
@@ -508,20 +519,10 @@ int enqueue_linear(ihip_ctx* c, const LinearCall& k)
            (const int*)k.perm, k.x_per_slot, 0, (const float*)k.x, nullptr, 1, 0};
     if (k.items && k.item_rows > 64) return fail(IHIP_E_ARG, "EnqueueLinear: items of at most 64 slots");
     char gname[32];
-    const bool flt32 = float_fmt(k.dtype) && !k.items && k.rows <= 32;
-    const int64_t bm = flt32 ? 32 : 64;
     snprintf(gname, sizeof gname, "gemm_%s_r%d", fmt_name(k.dtype), (int)bm);
     const unsigned gx = (unsigned)((k.out + 4096 / bm - 1) / (4096 / bm));
     const unsigned gy = (unsigned)(k.items ? k.nitems : (k.rows + bm - 1) / bm);
-    // float weights with too few tiles to fill the chip (a router: 128
-    // outputs): the sum split into ksplit parts of >= 256 values, one block
-    // each, then their double sums added in split order
-    int ksplit = 1;
-    if (float_fmt(k.dtype) && !k.items && !k.no_alloc && !c->capturing && c->gemm_split) {
-      const int64_t tiles = (int64_t)gx * gy;
-      while (ksplit < 16 && tiles * ksplit * 2 <= (int64_t)c->cus * 2 && k.in / (ksplit * 2) >= 256)
-        ksplit *= 2;
-    }
+    const int ksplit = may_split ? flt_parts : 1;
     if (ksplit > 1) {
       const int64_t n = k.rows * k.out;
       int rc = scratch(c, c->scratch_split, c->scratch_split_bytes, (uint64_t)n * ksplit * 8);

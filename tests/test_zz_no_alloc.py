@@ -59,6 +59,35 @@ def test_static_matches_allocating_entry_point(ctx, dtype, mode):
         assert H.lib().ihip_forget_weights(ctx.h, H._p(a), C.c_void_p(a.ctypes.data + a.nbytes)) >= 0
 
 
+# float weights: matrices whose sum the GEMM leaves whole (both entry points run
+# it: the same bits) and splits (only the allocating one may: the order of a
+# double sum, at most one ulp of single in 1/1000 of the values)
+@pytest.mark.parametrize("dtype", [H.F32, H.BF16, H.F16])
+@pytest.mark.parametrize("nin,out,whole", [(512, 66000, True), (4096, 3100, False), (1024, 3100, False)])
+def test_static_float_batches(ctx, dtype, nin, out, whole):
+    w = H.synth_normal(dtype, out, nin, 78, 0.05)
+    wd = C.c_uint64()
+    H.check(H.lib().ihip_weight(ctx.h, H._p(w), dtype, out, nin, 1, C.byref(wd)), "weight")
+    rng = np.random.default_rng(dtype)
+    for rows in (15, 8, 4, 20):
+        x = rng.standard_normal((rows, nin)).astype(np.float32)
+        names = []
+        for fn in (H.lib().ihip_enqueue_linear_at_static, H.lib().ihip_enqueue_linear_at):
+            ctx.kernel_timer("ge", 16)
+            names.append(run(ctx, fn, x, wd.value, dtype, out, 0, H.MODE_Q8))
+            names.append(list(ctx.kernel_timer_report()))
+            ctx.kernel_timer(None)
+        a, ka, b, kb = names
+        if whole:
+            assert ka == kb and ka[0].startswith("gemm_"), (rows, ka, kb)
+            assert np.array_equal(a.view(np.uint32), b.view(np.uint32)), rows
+        bits = np.abs(a.view(np.int32).astype(np.int64) - b.view(np.int32).astype(np.int64))
+        # (a value within a rounding of zero may change its sign bit: compared by size)
+        assert np.all((bits <= 1) | (np.abs(a - b) <= np.abs(b) * 2.0 ** -23 + 1e-30)), rows
+        assert (bits > 0).mean() <= 1e-3, rows
+    assert H.lib().ihip_forget_weights(ctx.h, H._p(w), C.c_void_p(w.ctypes.data + w.nbytes)) >= 0
+
+
 def test_static_refuses_beyond_its_size(ctx):
     nin, out, dtype = 4096, 64, H.Q8_0
     rows = (8 << 20) // (nin + nin // 8) + 1  # one row more than the array holds
