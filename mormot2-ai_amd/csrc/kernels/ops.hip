@@ -1130,9 +1130,10 @@ extern "C" __global__ __launch_bounds__(256) void attention_rows_f32_128(AttnArg
 //
 // A key that a row of the tile does not see has weight 0 in it, and its value
 // meets that weight in the product: 0 only while it is finite, else a NaN. So a
-// block whose sums are not all finite forms them again (`odd`): its products then
-// leave out the values that are not finite, and each row that sees such a
-// value's key adds it on its own.
+// block whose sums are not all finite walks its ranges again, each row adding the
+// keys that it sees one by one. (Apart from the walk above: a choice
+// inside it costs its registers and lets the products wait for all the loads, 75 ->
+// 77 us for 1000 rows, a window of 128 and 64 heads of 64.)
 //
 // Bound by the f64 matrix cores (4 hd operations a row and key, a 64-cycle
 // MFMA per 2048: 111 of the 188 us below) and the vector instructions beside
@@ -1204,7 +1205,7 @@ __device__ __forceinline__ void attention_mfma_t(const AttnArgs& a)
   const int it0 = s * nit / a.splits, it1 = (s + 1) * nit / a.splits;
   constexpr int DQ = d / 4;  // scores: k steps = a lane's dimensions
   float qa[DQ];  // (widened at each use: as doubles they halve the waves a SIMD holds)
-  {
+  auto load_q = [&]() __attribute__((always_inline)) {
     const int qr = r0 + min(lc, rlast);
     const float4* qp = (const float4*)(a.q + (int64_t)qr * qw + (int64_t)h * d + lq * DQ);
 #pragma unroll
@@ -1215,26 +1216,24 @@ __device__ __forceinline__ void attention_mfma_t(const AttnArgs& a)
       qa[4 * i + 2] = u.z;
       qa[4 * i + 3] = u.w;
     }
-  }
+  };
+  load_q();
   constexpr int NT = d / 64;  // values: dimensions of a lane, one per tile
   constexpr uint32_t ES = F16 ? 2 : 4;
   const int dim0 = w * (d / 4) + NT * lc;
   dbl4 o[NT];
-  bool odd = false;
-again:
-  if (t < ATTM) {
-    stat[t][0] = -1.0e308;
-    stat[t][1] = 0.0;
-  }
+  auto begin = [&]() __attribute__((always_inline)) {
+    if (t < ATTM) {
+      stat[t][0] = -1.0e308;
+      stat[t][1] = 0.0;
+    }
 #pragma unroll
-  for (int n = 0; n < NT; n++) o[n] = dbl4{0.0, 0.0, 0.0, 0.0};
-  __syncthreads();
-  for (int it = it0; it < it1; it++) {
-    const int kb = kb0 + it * per, ke = min(kend, kb + per);
-    const int nblk = (ke - kb + 15) >> 4, nk = 16 * nblk;  // blocks of 16 keys (<= 9)
-    double (*p)[ATTMK + 1] = sc[it & 1];
-    // ---- scores: wave w takes key blocks w, w + 4, w + 8; lane group lq
-    // the dimensions [lq * d / 4, (lq + 1) * d / 4)
+    for (int n = 0; n < NT; n++) o[n] = dbl4{0.0, 0.0, 0.0, 0.0};
+    __syncthreads();
+  };
+  // ---- scores: wave w takes key blocks w, w + 4, w + 8; lane group lq
+  // the dimensions [lq * d / 4, (lq + 1) * d / 4)
+  auto scores = [&](double (*p)[ATTMK + 1], int kb, int ke, int nblk) __attribute__((always_inline)) {
     for (int kbk = w; kbk < nblk; kbk += 4) {
       const int key = min(kb + 16 * kbk + lc, ke - 1);
       const int64_t kr = (int64_t)key * kvw + (int64_t)g * d + lq * DQ;
@@ -1268,103 +1267,106 @@ again:
         p[r][16 * kbk + lc] = in ? acc[v] * a.scale : -1.0e308;
       }
     }
-    __syncthreads();
-    // ---- per row: the new maximum, the weights exp(score - max), the sum
-    // (row 4 w + lq over the 16 lanes of its lane group, all rows at once)
-    {
-      constexpr int NB = ATTMK / 16;
-      double* pr = p[4 * w + lq] + lc;
-      const double old = stat[4 * w + lq][0];
-      double x[NB], m = old;
+  };
+  // ---- per row: the new maximum, the weights exp(score - max), the sum
+  // (row 4 w + lq over the 16 lanes of its lane group, all rows at once)
+  auto weights = [&](double (*p)[ATTMK + 1], int nblk) __attribute__((always_inline)) {
+    constexpr int NB = ATTMK / 16;
+    double* pr = p[4 * w + lq] + lc;
+    const double old = stat[4 * w + lq][0];
+    double x[NB], m = old;
 #pragma unroll
-      for (int i = 0; i < NB; i++) {
-        x[i] = i < nblk ? pr[16 * i] : -1.0e308;
-        m = fmax(m, x[i]);
+    for (int i = 0; i < NB; i++) {
+      x[i] = i < nblk ? pr[16 * i] : -1.0e308;
+      m = fmax(m, x[i]);
+    }
+    m = fmax(m, xpart<1>(m));
+    m = fmax(m, xpart<2>(m));
+    m = fmax(m, xpart<4>(m));
+    m = fmax(m, xpart<8>(m));
+    double e = 0;
+#pragma unroll
+    for (int i = 0; i < NB; i++)
+      if (i < nblk) {
+        // (a NaN score stays one, as in the CPU's sum)
+        const double y = x[i] == -1.0e308 ? 0.0 : exp_below(x[i] - m);
+        pr[16 * i] = y;
+        e += y;
       }
-      m = fmax(m, xpart<1>(m));
-      m = fmax(m, xpart<2>(m));
-      m = fmax(m, xpart<4>(m));
-      m = fmax(m, xpart<8>(m));
-      double e = 0;
+    e = wave_sum(e, 16);
+    if (lc == 0) {
+      const double f = old > -1.0e308 ? exp_below(old - m) : 0.0;
+      shrink[4 * w + lq] = f;
+      stat[4 * w + lq][0] = m;
+      stat[4 * w + lq][1] = __builtin_fma(stat[4 * w + lq][1], f, e);
+    }
+  };
+  auto shrunk = [&]() __attribute__((always_inline)) {
 #pragma unroll
-      for (int i = 0; i < NB; i++)
-        if (i < nblk) {
-          // (a NaN score stays one, as in the CPU's sum)
-          const double y = x[i] == -1.0e308 ? 0.0 : exp_below(x[i] - m);
-          pr[16 * i] = y;
-          e += y;
+    for (int v = 0; v < 4; v++) {
+      const double f = shrink[lq + 4 * v];
+#pragma unroll
+      for (int n = 0; n < NT; n++) o[n][v] *= f;
+    }
+  };
+  // this lane's values of key k of the range at vbase (past the last: the last): a
+  // uniform base and 24-bit products for the lane's offset (a range is at most
+  // ATTMK rows of kvw values)
+  const uint32_t vrow = (uint32_t)kvw * ES, vdim = (uint32_t)dim0 * ES;
+  auto values = [&](const uint8_t* vbase, uint32_t vlast, uint32_t k, float (&v)[NT]) __attribute__((always_inline)) {
+    const uint8_t* vp = vbase + (__umul24(min(k, vlast), vrow) + vdim);
+    if constexpr (F16) {
+      if constexpr (NT == 1) {
+        v[0] = half_to_float(*(const uint16_t*)vp);
+      } else {
+        uint32_t x[NT / 2];
+        if constexpr (NT == 2) {
+          x[0] = *(const uint32_t*)vp;
+        } else {
+          const uint2 y = *(const uint2*)vp;
+          x[0] = y.x;
+          x[1] = y.y;
         }
-      e = wave_sum(e, 16);
-      if (lc == 0) {
-        const double f = old > -1.0e308 ? exp_below(old - m) : 0.0;
-        shrink[4 * w + lq] = f;
-        stat[4 * w + lq][0] = m;
-        stat[4 * w + lq][1] = __builtin_fma(stat[4 * w + lq][1], f, e);
+#pragma unroll
+        for (int n = 0; n < NT; n++) v[n] = half_to_float((n & 1) ? x[n / 2] >> 16 : x[n / 2] & 0xffffu);
+      }
+    } else {
+      if constexpr (NT == 1) {
+        v[0] = *(const float*)vp;
+      } else if constexpr (NT == 2) {
+        const float2 x = *(const float2*)vp;
+        v[0] = x.x;
+        v[1] = x.y;
+      } else {
+        const float4 x = *(const float4*)vp;
+        v[0] = x.x;
+        v[1] = x.y;
+        v[2] = x.z;
+        v[3] = x.w;
       }
     }
+  };
+  begin();
+  for (int it = it0; it < it1; it++) {
+    const int kb = kb0 + it * per, ke = min(kend, kb + per);
+    const int nblk = (ke - kb + 15) >> 4, nk = 16 * nblk;  // blocks of 16 keys (<= 9)
+    double (*p)[ATTMK + 1] = sc[it & 1];
+    scores(p, kb, ke, nblk);
+    __syncthreads();
+    weights(p, nblk);
     __syncthreads();
     // ---- the weighted values: wave w the dimensions [w * d / 4, (w + 1) *
     // d / 4) as NT tiles of 16 (the wave's dimensions modulo NT); lane group
     // lq the range's keys [lq * S, (lq + 1) * S)
-    if (it > it0) {
-#pragma unroll
-      for (int v = 0; v < 4; v++) {
-        const double f = shrink[lq + 4 * v];
-#pragma unroll
-        for (int n = 0; n < NT; n++) o[n][v] *= f;
-      }
-    }
+    if (it > it0) shrunk();
     const int S = nk >> 2;  // k steps (nk is a multiple of 16)
     constexpr int VU = NT > 2 ? 4 : 12;  // value loads in flight per lane
-    // a uniform base and 24-bit products for the lane's offset (a range is at
-    // most ATTMK rows of kvw values)
     const uint8_t* vbase = (const uint8_t*)a.vc + ((int64_t)kb * kvw + (int64_t)g * d) * ES;
-    const uint32_t vlast = (uint32_t)(ke - 1 - kb), vrow = (uint32_t)kvw * ES, vdim = (uint32_t)dim0 * ES;
-    // this lane's values of key k of the range (past the last: the last)
-    auto values = [&](uint32_t k, float (&v)[NT]) __attribute__((always_inline)) {
-      const uint8_t* vp = vbase + (__umul24(min(k, vlast), vrow) + vdim);
-      if constexpr (F16) {
-        if constexpr (NT == 1) {
-          v[0] = half_to_float(*(const uint16_t*)vp);
-        } else {
-          uint32_t x[NT / 2];
-          if constexpr (NT == 2) {
-            x[0] = *(const uint32_t*)vp;
-          } else {
-            const uint2 y = *(const uint2*)vp;
-            x[0] = y.x;
-            x[1] = y.y;
-          }
-#pragma unroll
-          for (int n = 0; n < NT; n++) v[n] = half_to_float((n & 1) ? x[n / 2] >> 16 : x[n / 2] & 0xffffu);
-        }
-      } else {
-        if constexpr (NT == 1) {
-          v[0] = *(const float*)vp;
-        } else if constexpr (NT == 2) {
-          const float2 x = *(const float2*)vp;
-          v[0] = x.x;
-          v[1] = x.y;
-        } else {
-          const float4 x = *(const float4*)vp;
-          v[0] = x.x;
-          v[1] = x.y;
-          v[2] = x.z;
-          v[3] = x.w;
-        }
-      }
-    };
-    auto finite = [](float v) __attribute__((always_inline)) { return (float_bits(v) & 0x7f800000u) != 0x7f800000u; };
+    const uint32_t vlast = (uint32_t)(ke - 1 - kb);
     for (int t0 = 0; t0 < S; t0 += VU) {
       float vv[VU][NT];
 #pragma unroll
-      for (int u = 0; u < VU; u++) values(lq * S + t0 + u, vv[u]);
-      if (odd) {
-#pragma unroll
-        for (int u = 0; u < VU; u++)
-#pragma unroll
-          for (int n = 0; n < NT; n++) vv[u][n] = finite(vv[u][n]) ? vv[u][n] : 0.f;
-      }
+      for (int u = 0; u < VU; u++) values(vbase, vlast, lq * S + t0 + u, vv[u]);
 #pragma unroll
       for (int u = 0; u < VU; u++) {
         if (t0 + u < S) {
@@ -1375,33 +1377,39 @@ again:
         }
       }
     }
-    if (odd) {
+  }
+  bool bad = false;
+#pragma unroll
+  for (int n = 0; n < NT; n++)
+#pragma unroll
+    for (int v = 0; v < 4; v++) bad |= !__builtin_isfinite(o[n][v]);
+  const bool any = __any(bad);
+  if (l == 0) odds[w] = any;
+  __syncthreads();
+  if (odds[0] | odds[1] | odds[2] | odds[3]) {
+    load_q();  // (held from above, q would cost the first walk its registers)
+    begin();
+    for (int it = it0; it < it1; it++) {
+      const int kb = kb0 + it * per, ke = min(kend, kb + per);
+      const int nblk = (ke - kb + 15) >> 4;
+      double (*p)[ATTMK + 1] = sc[it & 1];
+      scores(p, kb, ke, nblk);
+      __syncthreads();
+      weights(p, nblk);
+      __syncthreads();
+      if (it > it0) shrunk();
+      const uint8_t* vbase = (const uint8_t*)a.vc + ((int64_t)kb * kvw + (int64_t)g * d) * ES;
       for (int k = 0; k < ke - kb; k++) {
         float x[NT];
-        values(k, x);
+        values(vbase, (uint32_t)(ke - 1 - kb), k, x);
 #pragma unroll
-        for (int n = 0; n < NT; n++)
-          if (!finite(x[n]))
+        for (int v = 0; v < 4; v++) {
+          const int r = lq + 4 * v;
+          if (kb + k >= first(r) && kb + k <= past + r0 + r)
 #pragma unroll
-            for (int v = 0; v < 4; v++) {
-              const int r = lq + 4 * v;
-              if (kb + k >= first(r) && kb + k <= past + r0 + r) o[n][v] = __builtin_fma(p[r][k], (double)x[n], o[n][v]);
-            }
+            for (int n = 0; n < NT; n++) o[n][v] = __builtin_fma(p[r][k], (double)x[n], o[n][v]);
+        }
       }
-    }
-  }
-  if (!odd) {
-    bool bad = false;
-#pragma unroll
-    for (int n = 0; n < NT; n++)
-#pragma unroll
-      for (int v = 0; v < 4; v++) bad |= !(fabs(o[n][v]) <= 1.7976931348623157e308);
-    const bool any = __any(bad);
-    if (l == 0) odds[w] = any;
-    __syncthreads();
-    if (odds[0] | odds[1] | odds[2] | odds[3]) {
-      odd = true;
-      goto again;
     }
   }
   // ---- row lq + 4 v, dimension(s) dim0 + n: the output, or the partial sums
