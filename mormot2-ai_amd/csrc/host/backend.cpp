@@ -363,6 +363,37 @@ bool gemm_runs(const ihip_ctx* c, int dtype, int mode)
   return c->use_gemm && (mode & 1) == IHIP_MODE_Q8 && gemm_fmt(dtype);
 }
 
+// the (8 rows, output)s from which 9 to 79 quantized rows take the GEMM. The 8-row
+// launches' time is flat at first and then grows with rows x outputs x groups of
+// the sum, the GEMM's with the chunks of a part of the sum while its tiles fit the
+// chip, so the line hardly depends on the sum; it does on how the launches cut a
+// row (U groups a lane: 3 of short sums run well, 4 poorly; an odd number of
+// groups of Q4_0, Q5_0 and Q5_1 is read unaligned) and on the GEMM's work a group
+// (Q5_1's second term, Q6_K's two products). A sum of two chunks is one step of the
+// GEMM, faster at once but for these two types. Both sides timed for 7 types x 22
+// sums of 256 .. 8192 x 10 output counts x 10 or 13 row counts (us a call with its
+// quantizer, 8-row launches / GEMM: 16 rows of 2048 -> 6144 Q4_K 15.3 / 9.9, Q6_K
+// 16.4 / 11.5; 24 of 1024 -> 3072 Q4_0 9.7 / 7.8; 9 of 256 -> 2048 Q4_0 7.6 / 7.0; 28 of
+// 1376 -> 2304 Q4_0 20.3 / 10.2; left to the launches: 9 of 2048 -> 3072 Q4_0 9.1 / 9.4,
+// 17 of 1024 -> 2048 Q6_K 8.0 / 8.9, 9 of 4096 -> 1024 Q4_0 8.6 / 14.5): over the 15630
+// shapes the mean time is 0.3% above that of always taking the faster side, 0.5% of
+// them are over 10% above it; with one line of 6144 for all 1.4% and 5.1%.
+static int64_t gemm_line(int dtype, int64_t G, int U)
+{
+  if ((G & 1) && (dtype == DT_Q4_0 || dtype == DT_Q5_0 || dtype == DT_Q5_1)) return G <= 16 ? 0 : 3712;
+  // Q4_0, Q5_0, Q4_K / Q8_0, MXFP4 / Q5_1 / Q6_K
+  const int t = dtype == DT_Q6_K ? 3 : dtype == DT_Q5_1 ? 2 : dtype == DT_Q8_0 || dtype == DT_MXFP4 ? 1 : 0;
+  static const int two_chunks[4] = {0, 0, 8832, 17024}, u1_short[4] = {3968, 2048, 4864, 8704},
+                   u1[4] = {4864, 4608, 5888, 6400}, u2[4] = {5120, 6784, 6784, 8320},
+                   u3_short[4] = {7808, 7808, 8832, 10752}, u3[4] = {5120, 5120, 8064, 6400},
+                   u4[4] = {3584, 4736, 4480, 4736}, u4_long[4] = {3584, 3840, 4992, 3712};
+  if (G <= 16) return two_chunks[t];
+  if (U == 1) return (G < 48 ? u1_short : u1)[t];
+  if (U == 2) return u2[t];
+  if (U == 3) return (G < 64 ? u3_short : u3)[t];
+  return (G <= 128 ? u4 : u4_long)[t];
+}
+
 int enqueue_linear(ihip_ctx* c, const LinearCall& k)
 {
   if (!linear_ok(k.dtype, k.in) || k.out < 1 || k.out > INT32_MAX || k.rows < 1 || k.rows > 65535 ||
@@ -458,23 +489,14 @@ int enqueue_linear(ihip_ctx* c, const LinearCall& k)
                k.rk > std::min<int64_t>(k.rexp, 8) || k.rk != k.rows))
     return fail(IHIP_E_ARG, "EnqueueLinear: self-routing takes one token's <= 8 slots of <= 256 experts, gate/up with a norm or a quantized row");
   if (k.w2 && batch) return fail(IHIP_E_ARG, "EnqueueLinear: the fused SwiGLU takes one row per block");
-  // a chunk of rows in the Q8 arithmetic: the MFMA GEMM (64 x 64 tiles)
-  // (float weights in the Q8 arithmetic: the float activations as they are,
-  // on the f64 matrix cores)
+  // a chunk of rows in the Q8 arithmetic: the MFMA GEMM (blocks of 32 or 64 rows
+  // by 32 to 128 outputs; float weights in the Q8 arithmetic: the float
+  // activations as they are, on the f64 matrix cores)
   const bool gemm_q8 = (q8 || float_fmt(k.dtype)) && gemm_runs(c, k.dtype, mode);
   if (k.items && k.item_rows > 8 && !gemm_q8)
     return fail(IHIP_E_ARG, "EnqueueLinear: items of more than 8 slots need the GEMM");
   const int min_rows = float_fmt(k.dtype) ? c->gemm_min_rows_float : c->gemm_min_rows;
-  // quantized weights, fewer rows than that: the 8-row launches' time grows
-  // with the (8 rows, output, group)s, the GEMM's with the chunks of a part of
-  // the sum, and it needs enough (8 rows, output)s to fill the chip. The lines
-  // are the lowest at which none of 7 types x 9 sums of 256 .. 8192 x 12 output
-  // counts x 13 row counts runs over 6% slower than the 8-row launches, but one
-  // Q8_0 shape (12%); Q6_K's two products a group and Q5_1's second term pay
-  // later (us, 8-row launches / GEMM: 16 rows of 2048 -> 6144 Q4_K 14.3 / 8.8, Q6_K
-  // 14.9 / 10.1; 24 of 8192 -> 2048 Q4_K 49.3 / 21.0; left to the launches: 9 of 2048 ->
-  // 3072 Q5_1 9.5 / 11.3, 9 of 2048 -> 4096 Q8_0 8.0 / 10.0, 17 of 2048 -> 2048 Q6_K
-  // 8.1 / 10.0)
+  // quantized weights, 9 rows and more below that: gemm_line
   // float weights: the 8-row launches' time grows with rows x weights, the
   // GEMM's first 32 rows cost one tile (BF16, us, launches / GEMM: 4 rows of
   // 2048 -> 6144 38.9 / 30.1, 2 rows 21 / 30; 8 rows of 3072 -> 1024 29.9 /
@@ -493,11 +515,9 @@ int enqueue_linear(ihip_ctx* c, const LinearCall& k)
     while (flt_parts < 16 && tiles * flt_parts * 2 <= (int64_t)c->cus * 2 && k.in / (flt_parts * 2) >= 256)
       flt_parts *= 2;
   }
-  const int64_t elems = k.in * k.out, outs8 = (k.rows + 7) / 8 * k.out;
+  const int64_t elems = k.in * k.out;
   const bool few =
-      q8 ? c->gemm_few_rows && k.rows > 8 &&
-               ((outs8 >= 9216 && outs8 * G >= (k.dtype == DT_Q6_K || k.dtype == DT_Q5_1 ? 500000 : 400000)) ||
-                (outs8 >= 6144 && outs8 * G >= 1500000 && k.dtype != DT_Q5_1))
+      q8 ? c->gemm_few_rows && k.rows > 8 && k.rows * k.out >= 8 * gemm_line(k.dtype, G, U)
          : c->gemm_few_float && (may_split || flt_parts == 1) &&
                ((k.rows >= 4 && elems >= 12 << 20) || (k.rows >= 8 && elems >= 3 << 20));
   if (batch && gemm_q8 && (k.items ? k.item_rows > 8 : k.rows >= min_rows || few)) {
