@@ -15,9 +15,9 @@
 
 namespace ihip {
 
-// rows from which a Q8 Linear runs on the MFMA GEMM instead of 8-row GEMVs:
-// below 80 rows the GEMVs are faster (a 32-token prompt of Qwen3-0.6B
-// prefills 1.6x faster on them, a 128-token one 7% slower)
+// rows from which a Q8 Linear runs on the MFMA GEMM whatever its matrix; 9 to 79
+// rows do where the matrix and the sum are large enough (enqueue_linear's
+// `few`), the others on the 8-row launches
 constexpr int GEMM_MIN_ROWS = 80;
 // F32/BF16/F16 weights on the f64 GEMM from 16 rows: gpt-oss-20b's BF16
 // attention matrices take 19.3 ms for a 32-token prefill there against 25.0

@@ -6,7 +6,9 @@
 // quantized activation rows x (Q8_0 or Q8_K, by quantize_q8_0/_k) and weights
 // in the HIP layout of layout.h - the same terms, in double, as the one-row
 // GEMV of linear.hip (group_q8, group_q8k, superblock_q8k); only the order of
-// the double sum over groups differs (here: group order).
+// the double sum over groups differs (here: group order, or with a block's KS
+// waves sharing the sum, wave k the chunks of 8 groups k, k + KS, .. in order
+// and then the waves' sums in wave order).
 //
 // Mapping to CDNA4: a wave owns one or two tiles of 32 rows x 32 outputs. Per
 // 32-value group it runs v_mfma_i32_32x32x32_i8 with A = the activation codes
@@ -24,12 +26,13 @@
 // values 8h..8h+7 of each: with the group's nibble order (byte j: value j,
 // value j + 16) both come from bytes 8h..8h+7 of the 16-byte group.
 //
-// Bound by the vector unit and the chain LDS -> widening -> MFMA -> terms of
-// a group, which two or three waves a SIMD cover; 41 (Q4_K) to 60 vector
-// instructions per tile and group. Measured against the 64 x 64 tiles with
-// row scales in LDS that this replaces, us: Q4_K 512 rows 2048 -> 6144
-// 47.5 -> 31.9 (403 TOP/s), 1024 rows 2048 -> 4096 37.4 (459), Q6_K 512 rows
-// 60 -> 51, Q8_0 301 rows 3072 -> 1024 34.7 -> 17.5 (the sum over 4 waves).
+// Bound by the chain LDS -> widening -> MFMA -> terms of a group and the two
+// barriers of a step, which two waves a SIMD do not cover: on full chips vector
+// instructions issue 45% of the time (36 to 59 per MFMA), MFMAs 9%. Measured
+// against the 64 x 64 tiles with row scales in LDS that this replaces, us, the
+// launch alone: Q4_K 512 rows 2048 -> 6144 47.8 -> 30.4 (424 TOP/s), 1024 rows
+// 2048 -> 4096 61.9 -> 34.0 (505), Q6_K 512 rows 58.8 -> 47.2, Q8_0 51.9 -> 43.7,
+// 301 rows 3072 -> 1024 35.4 -> 16.7 (the sum over 4 waves).
 //
 // Operand layout of both MFMAs (probed on gfx950): A lane l = row l % 32,
 // B lane l = column l % 32, 16 (8) k values each, the k order free but the
@@ -704,7 +707,8 @@ __device__ __forceinline__ void gemm_tiles(const GemmArgs& a, const uint8_t* wb,
 #pragma unroll
         for (int m = 0; m < MT; m++) {
           terms(j, m, s[m], x);
-          // (free to move them further, the scheduler would spill)
+          // (free to move them further, the scheduler would spill; Q6_K's
+          // 64-row tile, at 256 registers, holds 11 in scratch even so)
           __builtin_amdgcn_sched_barrier(0);
         }
       }
@@ -1079,9 +1083,9 @@ __device__ __forceinline__ void gemm8(const GemmArgs& a)
 //
 // A lane group's k values are a contiguous quarter of the chunk, so a lane
 // reads its 8 steps of a tile row as two 16-byte LDS words. Bound by the f64
-// matrix cores (a 64-cycle MFMA per 1024 products: 307 of the 717 us of 1024
+// matrix cores (a 64-cycle MFMA per 1024 products: 307 of the 714 us of 1024
 // rows 2880 -> 4096 before, when the operands came by 4-byte loads and LDS
-// reads; 442 now). 32 rows x 128 outputs for up to 32 rows, whose
+// reads; 397 now). 32 rows x 128 outputs for up to 32 rows, whose
 // matrix work is half a 64-row tile's.
 typedef double v4d __attribute__((ext_vector_type(4)));
 constexpr int FKC = 32;       // values of the sum per chunk

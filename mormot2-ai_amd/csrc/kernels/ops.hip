@@ -191,8 +191,9 @@ struct NormArgs {
 // cd: x += the expert rows weighted in slot order, each step single-rounded
 // as TDecoderModel.Experts adds them (decoder.pas:3140-3148)
 // One block of 1024 per row; a thread keeps its NV columns c = t + 1024 i in
-// registers and issues all their loads (and those of the k expert rows)
-// before the first sum, so a row costs one memory round trip.
+// registers and issues all their loads before the first sum, so a row costs
+// one memory round trip; k expert rows are loaded and added 8 at a time, one
+// round trip more for each further 8.
 #define NORM_NV 4
 extern "C" __global__ __launch_bounds__(1024, 8) void rmsnorm(NormArgs a)
 {
@@ -1131,9 +1132,9 @@ extern "C" __global__ __launch_bounds__(256) void attention_rows_f32_128(AttnArg
 // A key that a row of the tile does not see has weight 0 in it, and its value
 // meets that weight in the product: 0 only while it is finite, else a NaN. So a
 // block whose sums are not all finite walks its ranges again, each row adding the
-// keys that it sees one by one. (Apart from the walk above: a choice
-// inside it costs its registers and lets the products wait for all the loads, 75 ->
-// 77 us for 1000 rows, a window of 128 and 64 heads of 64.)
+// keys that it sees one by one. (In code of its own: a choice inside the ordinary
+// walk costs registers and lets its products wait for all the loads, 75 -> 77 us
+// for 1000 rows, a window of 128 and 64 heads of 64.)
 //
 // Bound by the f64 matrix cores (4 hd operations a row and key, a 64-cycle
 // MFMA per 2048: 111 of the 188 us below) and the vector instructions beside
