@@ -1308,18 +1308,31 @@ int enqueue_attention_one(ihip_ctx* c, const AttnOne& o)
 }
 
 // the groups that the key ranges of `tiles` (head, 16 rows) tiles are shared
-// between, each a block: one, with no merge, where the tiles give every CU two
-// blocks or there are two ranges at most and enough rows that the merge costs
-// more than a block's second range (32 heads of 128, 100 rows after 60: 25.5 us in two
-// groups, 13.4 in one); else as many as give every CU two, or one more where the
-// fullest CU then walks fewer ranges (16 heads of 128, 100 rows after 2000: 112 tiles, 17
-// ranges: 5 groups 75.2 us, 6 groups 63.8)
-static int attention_groups(int64_t tiles, int64_t heads, int64_t rows, int64_t splits, int64_t cus)
+// between, each a block. One, with no merge, where the tiles give every CU two
+// blocks, where a tile's keys are one piece, and where the merge of the rows
+// costs more than the few ranges that a block walks on its own (32 heads of 128, 100
+// rows after 60: 28.3 us in two groups, 15.8 in one; 16 heads, 250 rows after 60 31.9,
+// 23.2): of two ranges from a number of (head, row)s - later where the second is
+// not short, and for heads of 256, whose ranges take longer - of three from 3 / 5
+// of a tile a CU, of five from one. Else as many as reside at once, so that none
+// waits for a second round (112 tiles of heads of 256, 17 ranges: 5 groups 135.8 us, 4
+// 108.4; 96 of heads of 128: 6 groups 58.7, 8 48.5), of heads of 128 the fewest with as
+// short a walk (112 tiles, 8 ranges: 6 groups 45.0, 4 40.5); up to four ranges of
+// heads of 256, which end at different times, one more. Over 2362 shapes the mean
+// time is 0.8% above that of the best number of groups, at most 20% (as many as
+// give every CU two blocks: 4.7%, 99%).
+static int attention_groups(int64_t tiles, int64_t heads, int64_t rows, int64_t hd, int64_t keys, int64_t splits,
+                            int64_t cus)
 {
-  if (tiles >= 2 * cus || (splits <= 2 && heads * rows >= 4 * cus)) return 1;
-  const auto ranges = [&](int64_t g) { return (tiles * g + cus - 1) / cus * ((splits + g - 1) / g); };
-  const int64_t g = std::min(splits, (2 * cus + tiles - 1) / tiles);
-  return (int)(g < splits && 2 * tiles * (g + 1) <= 7 * cus && ranges(g + 1) < ranges(g) ? g + 1 : g);
+  const int64_t alone = hd == 256 ? (keys <= 192 ? 2 * cus : 8 * cus) : keys <= 192 ? 3 * cus / 2 : 5 * cus;
+  if (tiles >= 2 * cus || keys <= 144 || (splits <= 2 && heads * rows >= alone) ||
+      (splits <= 3 && 5 * tiles >= 3 * cus) || (splits <= 5 && tiles >= cus))
+    return 1;
+  const int64_t resident = cus * (hd == 64 ? 4 : hd == 128 ? 3 : 2);  // blocks of the kernels
+  int64_t g = hd == 256 && splits <= 4 ? (resident + tiles - 1) / tiles : resident / tiles;
+  g = std::min(splits, std::max<int64_t>(2, g));
+  const int64_t walk = (splits + g - 1) / g;  // ranges of the longest group
+  return (int)(hd == 128 ? (splits + walk - 1) / walk : g);
 }
 
 int enqueue_attention(ihip_ctx* c, uint64_t q, uint64_t kc, uint64_t vc, uint64_t y, uint64_t part,
@@ -1345,17 +1358,18 @@ int enqueue_attention(ihip_ctx* c, uint64_t q, uint64_t kc, uint64_t vc, uint64_
   int rc;
   // few rows of half-float heads of 256: a block of the tiles below walks 16
   // rows of a range however few there are, 19 us at best, where attention_part's
-  // blocks, one per row and range, take 16 while they fit in one or two rounds
+  // blocks, one per row and range, take 16 while no CU has more than two
   // (8 heads: 8 rows after 500 16.5 us there, 19.9 in tiles; 8 rows after 2000 in a window
   // of 1024 19.9, 24.3; 32 rows after 500 29.3, 21.4; float keys are slower there at once)
   const int64_t keys = window > 0 ? std::min(past + rows, window) : past + rows, blocks = heads * rows * splits;
   const bool few = hd == 256 && f16 &&
-                   (splits == 1 ? keys >= 72 && blocks <= c->cus : 2 * blocks <= (splits <= 8 ? 5 : 4) * c->cus);
+                   (splits == 1 ? keys >= 72 && blocks <= c->cus : blocks <= 2 * c->cus);
   if ((hd == 64 || hd == 128 || hd == 256) && rows > 1 && c->attn_mfma && kvh * hd < 1 << 22 && !few) {
     // tiles of 16 rows on the f64 matrix cores, a block per tile, head and group
     // of the tile's key ranges; the offsets inside a range are 24-bit products
     // of its rows' bytes
-    const int groups = attention_groups(heads * ((rows + 15) / 16), heads, rows, splits, c->cus);
+    const int groups = attention_groups(heads * ((rows + 15) / 16), heads, rows, hd, window > 0 ? keys + 15 : keys,
+                                        splits, c->cus);
     a.splits = groups;
     char name[32];
     snprintf(name, sizeof name, "attention_mfma_%s_%d", f16 ? "f16" : "f32", (int)hd);

@@ -61,7 +61,11 @@ def test_tiles_match_oracle(ctx, heads, kvh, hd, rows, past, window, sinks, half
 # of 256)
 ROUTES = [
     (32, 4, 128, 100, 60, 0, True, "mfma"), (14, 2, 64, 200, 0, 0, False, "mfma"),
-    (8, 2, 128, 100, 60, 0, True, "mfma merge"), (16, 8, 128, 100, 2000, 0, True, "mfma merge"),
+    (8, 2, 128, 100, 60, 0, True, "mfma"), (8, 2, 128, 33, 200, 0, True, "mfma merge"),
+    (4, 2, 128, 20, 120, 0, False, "mfma"), (16, 8, 128, 100, 2000, 0, True, "mfma merge"),
+    (16, 8, 128, 250, 60, 0, True, "mfma"), (8, 2, 256, 150, 2000, 0, True, "mfma merge"),
+    (16, 8, 256, 250, 400, 0, False, "mfma merge"), (14, 2, 64, 20, 400, 128, True, "mfma"),
+    (4, 2, 64, 20, 700, 300, True, "mfma merge"), (16, 8, 256, 10, 500, 0, True, "mfma merge"),
     (14, 2, 64, 300, 2000, 0, True, "mfma merge"), (8, 2, 256, 8, 500, 0, True, "part merge"),
     (8, 2, 256, 8, 500, 0, False, "mfma merge"), (8, 2, 256, 8, 2000, 1024, True, "part merge"),
     (8, 2, 256, 16, 2000, 128, True, "part merge"), (8, 2, 256, 64, 60, 0, True, "mfma"),
